@@ -20,7 +20,7 @@ CSRC = PACKAGE / "csrc"
 BUILD = PACKAGE / "_build"
 LIBRARY = PACKAGE / "libflashim_amd.so"
 HOST_LIBRARY = PACKAGE / "libfim_host.so"
-DEVICE_SOURCES = ("quantize.hip", "igemm.hip", "depthwise.hip", "dwpw.hip", "mlp.hip", "stem.hip", "pointwise.hip", "version.hip")
+DEVICE_SOURCES = ("quantize.hip", "igemm.hip", "deep_plan.hip", "deep_int8.hip", "deep_mx.hip", "depthwise.hip", "dwpw.hip", "mlp.hip", "stem.hip", "pointwise.hip", "version.hip")
 PROBE_LIBRARY = PACKAGE / "libflashim_amd_probe.so"
 PROBE_SOURCES = ("probe.hip",)
 ARCH = os.environ.get("FLASHIM_AMD_ARCH", "gfx950")
