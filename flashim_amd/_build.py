@@ -1,7 +1,9 @@
 """Ahead-of-time build of the HIP library (``libflashim_amd.so``, gfx950) and of the host build of its scalar numerics
 (``libfim_host.so``, used by the CPU tests), and the device probes the tests and the bench use
-(``libflashim_amd_probe.so``: numerics hooks and an MFMA microbenchmark, kept out of the product library). The libraries are built in-tree so they travel with the source tree; the
-ctypes loader in :mod:`flashim_amd._lib` only loads what is built and never compiles at import time.
+(``libflashim_amd_probe.so``: numerics hooks and an MFMA microbenchmark, kept out of the product library), and the torch
+operators on top of the C ABI (``libflashim_amd_torch.so``). The libraries are built in-tree so they travel with the
+source tree; the loaders in :mod:`flashim_amd._lib` and :mod:`flashim_amd.library` only load what is built and never
+compile at import time.
 
 Flags: ``-ffp-contract=off`` keeps the epilogues' separate multiply and add roundings (the reference's order) unless a
 kernel asks for an FMA explicitly; ``-packed-fp32-ops`` is disabled for all device code.
@@ -23,6 +25,7 @@ HOST_LIBRARY = PACKAGE / "libfim_host.so"
 DEVICE_SOURCES = ("quantize.hip", "igemm.hip", "deep_plan.hip", "deep_int8.hip", "deep_mx.hip", "depthwise.hip", "dwpw.hip", "mlp.hip", "stem.hip", "pointwise.hip", "version.hip")
 PROBE_LIBRARY = PACKAGE / "libflashim_amd_probe.so"
 PROBE_SOURCES = ("probe.hip",)
+TORCH_LIBRARY = PACKAGE / "libflashim_amd_torch.so"
 ARCH = os.environ.get("FLASHIM_AMD_ARCH", "gfx950")
 HIP_FLAGS = (
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=off", "-munsafe-fp-atomics",
@@ -43,8 +46,25 @@ def _run(cmd: list[str]) -> None:
         raise RuntimeError(f"build step failed ({' '.join(cmd)}):\n{result.stderr[-4000:]}")
 
 
-def build(jobs: int = 4) -> Path:
-    """Compile every HIP source for gfx950 and link ``libflashim_amd.so``; build ``libfim_host.so``. Always rebuilds."""
+def build_torch_ops() -> Path:
+    """Compile ``csrc/torch_ops.cpp`` against the installed torch and link it to ``libflashim_amd.so`` beside it."""
+    import torch
+    from torch.utils import cpp_extension
+
+    temporary = TORCH_LIBRARY.with_suffix(f".{os.getpid()}.tmp")
+    torch_lib = Path(torch.__file__).parent / "lib"
+    includes = [flag for path in cpp_extension.include_paths("cuda") for flag in ("-isystem", path)]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, str(CSRC / "torch_ops.cpp"),
+          "-o", str(temporary), f"-L{PACKAGE}", "-lflashim_amd", f"-L{torch_lib}", "-lc10", "-ltorch_cpu", "-lc10_hip",
+          "-Wl,-rpath,$ORIGIN"])
+    temporary.replace(TORCH_LIBRARY)
+    return TORCH_LIBRARY
+
+
+def build(jobs: int = 6) -> Path:
+    """Compile every HIP source for gfx950 and link ``libflashim_amd.so``; build the torch operators on it and
+    ``libfim_host.so``. Always rebuilds."""
     BUILD.mkdir(exist_ok=True)
     compiler = hipcc()
     sources = DEVICE_SOURCES + PROBE_SOURCES
@@ -57,6 +77,7 @@ def build(jobs: int = 4) -> Path:
         _run([compiler, "-shared", "-fPIC", f"--offload-arch={ARCH}", *(str(objects[s]) for s in srcs),
               "-o", str(temporary)])
         temporary.replace(library)
+    build_torch_ops()
     host_tmp = HOST_LIBRARY.with_suffix(f".{os.getpid()}.tmp")
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", str(CSRC / "numerics_host.cpp"), "-o", str(host_tmp)])
     host_tmp.replace(HOST_LIBRARY)

@@ -30,19 +30,31 @@ from flashim_amd.platforms import is_gfx950
 conv_output_size = library.conv_out_hw
 
 
-def _bias(bias: Tensor | None, device: torch.device) -> Tensor | None:
+def on_device(t: Tensor, device: torch.device, dtype: torch.dtype) -> Tensor:
+    """``t`` contiguous on ``device`` as ``dtype``; a tensor that is so already is returned without a torch call."""
+    if t.dtype != dtype or t.device != device:
+        t = t.to(device=device, dtype=dtype)
+    return t if t.is_contiguous() else t.contiguous()
+
+
+def packed(t: Tensor) -> Tensor:
+    return t if t.is_contiguous() else t.contiguous()
+
+
+def bias_on(bias: Tensor | None, device: torch.device) -> Tensor | None:
     """FP32 or BF16 ``[N]`` on ``device`` (other dtypes promoted to FP32), or ``None``."""
     if bias is None:
         return None
-    if bias.dtype not in (torch.float32, torch.bfloat16):
-        bias = bias.float()
-    return bias.to(device).contiguous()
+    return on_device(bias, device, bias.dtype if bias.dtype in (torch.float32, torch.bfloat16) else torch.float32)
 
 
-def _residual(residual: Tensor | None, device: torch.device, out_shape: tuple[int, int, int, int]) -> Tensor | None:
+def _out_shape(x: Tensor, weight: Tensor, *geometry: int) -> tuple[int, int, int, int]:
+    b, h, w, _ = x.shape
+    return (b, *conv_output_size(h, w, *geometry), weight.shape[0])
+
+
+def _residual(residual: Tensor, device: torch.device, out_shape: tuple[int, int, int, int]) -> Tensor:
     """The residual as the kernels read it: ``[B, Ho, Wo, <= Cout]`` FP32 or BF16, any strides."""
-    if residual is None:
-        return None
     if residual.ndim != 4 or tuple(residual.shape[:3]) != tuple(out_shape[:3]) or residual.shape[3] > out_shape[3]:
         raise ValueError(f"residual {tuple(residual.shape)} does not fit the output {tuple(out_shape)}")
     if residual.device != device:
@@ -53,7 +65,10 @@ def _residual(residual: Tensor | None, device: torch.device, out_shape: tuple[in
 
 
 def _scalar(t: Tensor, device) -> Tensor:
-    return t.to(device=device, dtype=torch.float32).reshape(1).contiguous()
+    """One FP32 value on ``device`` (any shape of one element: the kernels read its address)."""
+    if t.numel() != 1:
+        raise RuntimeError(f"expected one value, got shape {tuple(t.shape)}")
+    return on_device(t, device, torch.float32)
 
 
 def _same_scale(scale: Tensor, device) -> Tensor:
@@ -71,14 +86,13 @@ def int8_conv2d(
 ) -> Tensor:
     """``x`` int8 ``[B, H, W, Cin]`` (packed), ``weight`` int8 ``[Cout, kh*kw*Cin]`` (ky, kx, c) -> BF16
     ``[B, Ho, Wo, Cout]``, or int8 with ``out_scale``."""
-    b, h, w, _ = x.shape
-    cout = weight.shape[0]
-    ho, wo = conv_output_size(h, w, kh, kw, sh, sw, ph, pw, dh, dw)
+    device = x.device
+    if residual is not None:
+        residual = _residual(residual, device, _out_shape(x, weight, kh, kw, sh, sw, ph, pw, dh, dw))
     return library.int8_conv2d(
-        x.contiguous(), weight.contiguous(), _scalar(a_scale, x.device),
-        w_scale.to(device=x.device, dtype=torch.float32).contiguous(), _bias(bias, x.device),
-        kh, kw, sh, sw, ph, pw, dh, dw, bool(relu), bool(gelu), _residual(residual, x.device, (b, ho, wo, cout)),
-        None if out_scale is None else _scalar(out_scale, x.device))
+        packed(x), packed(weight), _scalar(a_scale, device), on_device(w_scale, device, torch.float32),
+        bias_on(bias, device), kh, kw, sh, sw, ph, pw, dh, dw, bool(relu), bool(gelu), residual,
+        None if out_scale is None else _scalar(out_scale, device))
 
 
 def int8_conv2d_maxpool(
@@ -88,9 +102,8 @@ def int8_conv2d_maxpool(
     """``(out, pooled)``: the BF16 ``[B, Ho, Wo, Cout]`` conv output and the INT8 ``[B, Ho/2, Wo/2, Cout]`` 2x2 max pool
     of it quantized with ``out_scale`` (``ops/conv.py:209-222``), the pool from the conv's epilogue."""
     return library.int8_conv2d_maxpool(
-        x.contiguous(), weight.contiguous(), _scalar(a_scale, x.device),
-        w_scale.to(device=x.device, dtype=torch.float32).contiguous(), _bias(bias, x.device),
-        kh, kw, sh, sw, ph, pw, dh, dw, bool(relu), _scalar(out_scale, x.device))
+        packed(x), packed(weight), _scalar(a_scale, x.device), on_device(w_scale, x.device, torch.float32),
+        bias_on(bias, x.device), kh, kw, sh, sw, ph, pw, dh, dw, bool(relu), _scalar(out_scale, x.device))
 
 
 def mxfp8_conv2d(
@@ -101,16 +114,15 @@ def mxfp8_conv2d(
     """``x`` E4M3 ``[B, H, W, Cin]`` (``Cin % 32 == 0``), ``channel_exponent`` int8 ``[Cin / 32]``, ``weight`` E4M3
     ``[Cout, kh*kw*Cin]`` with ``weight_exponent`` ``[Cout, kh*kw*Cin / 32]`` -> BF16 ``[B, Ho, Wo, Cout]``, or E4M3
     with ``out_exponent``."""
-    b, h, w, _ = x.shape
-    cout = weight.shape[0]
-    ho, wo = conv_output_size(h, w, kh, kw, sh, sw, ph, pw, dh, dw)
+    device = x.device
+    if residual is not None:
+        residual = _residual(residual, device, _out_shape(x, weight, kh, kw, sh, sw, ph, pw, dh, dw))
     if out_exponent is not None:
-        out_exponent = out_exponent.to(device=x.device, dtype=torch.int8).contiguous()
+        out_exponent = on_device(out_exponent, device, torch.int8)
     out = library.mxfp8_conv2d(
-        x.contiguous().view(torch.uint8), channel_exponent.to(device=x.device, dtype=torch.int8).contiguous(),
-        weight.contiguous().view(torch.uint8), weight_exponent.to(device=x.device, dtype=torch.int8).contiguous(),
-        _bias(bias, x.device), kh, kw, sh, sw, ph, pw, dh, dw, bool(relu), bool(gelu),
-        _residual(residual, x.device, (b, ho, wo, cout)), out_exponent)
+        packed(x), on_device(channel_exponent, device, torch.int8), packed(weight),
+        on_device(weight_exponent, device, torch.int8), bias_on(bias, device), kh, kw, sh, sw, ph, pw, dh, dw,
+        bool(relu), bool(gelu), residual, out_exponent)
     return out if out_exponent is None else out.view(torch.float8_e4m3fn)
 
 
@@ -122,13 +134,13 @@ def _nhwc_bf16(value: Tensor) -> Tensor:
     references do with ``value.to(torch.bfloat16)``)."""
     if value.dtype != torch.bfloat16:
         value = value.to(torch.bfloat16)
-    return value.permute(0, 2, 3, 1).contiguous()
+    return packed(value.permute(0, 2, 3, 1))
 
 
 def _dw_operands(value: Tensor, weight: Tensor, bias: Tensor) -> tuple[Tensor, Tensor, Tensor]:
     """BF16 NHWC input, BF16 weight, and the bias as given when it is FP32 or BF16 (the kernels read either; the
     BF16 -> FP32 widening is exact), else widened to FP32."""
-    return (_nhwc_bf16(value), weight.to(device=value.device, dtype=torch.bfloat16).contiguous(), _bias(bias, value.device))
+    return (_nhwc_bf16(value), on_device(weight, value.device, torch.bfloat16), bias_on(bias, value.device))
 
 
 def depthwise5x5_relu_mxfp8(value: Tensor, weight: Tensor, bias: Tensor) -> tuple[Tensor, Tensor]:
@@ -153,7 +165,7 @@ def depthwise5x5_gelu(value: Tensor, weight: Tensor, bias: Tensor, *, scale: Ten
     if scale is not None:
         return library.depthwise5x5(*operands, 1, library.DW_INT8, _scalar(scale, value.device), None)
     if exponent is not None:
-        e = exponent.to(device=value.device, dtype=torch.int8).contiguous()
+        e = on_device(exponent, value.device, torch.int8)
         return library.depthwise5x5(*operands, 1, library.DW_MX_STATIC, None, e).view(torch.float8_e4m3fn)
     return library.depthwise5x5(*operands, 1, library.DW_BF16, None, None)
 
@@ -201,8 +213,8 @@ def depthwise5x5_relu_pointwise(value: Tensor, dw_weight: Tensor, dw_bias: Tenso
     tensor), then the BF16 pointwise GEMM with FP32 accumulation and bias."""
     batch, _, height, width = value.shape
     hidden = library.depthwise5x5(*_dw_operands(value, dw_weight, dw_bias), 0, library.DW_BF16, None, None)
-    out = library.pointwise_bf16(hidden, pw_weight.to(device=value.device, dtype=torch.bfloat16).contiguous(),
-                                 _bias(pw_bias, value.device))
+    out = library.pointwise_bf16(hidden, on_device(pw_weight, value.device, torch.bfloat16),
+                                 bias_on(pw_bias, value.device))
     return out.reshape(batch, height, width, -1).permute(0, 3, 1, 2)
 
 
@@ -226,7 +238,7 @@ def pointwise_mxfp8_fused(value: Tensor, dw_weight: Tensor, dw_bias: Tensor, pw_
     x, dw_w, dw_b = _dw_operands(value, dw_weight, dw_bias)
     out = library.depthwise5x5_relu_pointwise_mxfp8(
         x, dw_w, dw_b, pw_weight.contiguous().view(torch.uint8),
-        pw_scale_u8.to(value.device).contiguous().view(torch.uint8), _bias(pw_bias, value.device))
+        pw_scale_u8.to(value.device).contiguous().view(torch.uint8), bias_on(pw_bias, value.device))
     return out.permute(0, 3, 1, 2)
 
 
@@ -240,7 +252,7 @@ def pointwise_mxfp8_composite(value: Tensor, dw_weight: Tensor, dw_bias: Tensor,
     # the weight's E8M0 bytes go to the GEMM as they are (no per-call conversion to signed exponents)
     w_e8m0 = pw_scale_u8.to(value.device).contiguous().view(torch.int8).reshape(n, k // 32)
     out = library.mxfp8_scaled_mm(codes, swizzled, pw_weight.contiguous().view(torch.uint8), w_e8m0,
-                                  _bias(pw_bias, value.device), True)
+                                  bias_on(pw_bias, value.device), True)
     return out.reshape(batch, height, width, n).permute(0, 3, 1, 2)
 
 
@@ -263,7 +275,7 @@ def pointwise_int8_fused(value: Tensor, dw_weight: Tensor, dw_bias: Tensor, pw_w
     x, dw_w, dw_b = _dw_operands(value, dw_weight, dw_bias)
     out = library.depthwise5x5_relu_pointwise_int8(
         x, dw_w, dw_b, _scalar(scale, value.device), pw_weight.to(value.device).contiguous(),
-        pw_wscale.to(device=value.device, dtype=torch.float32).contiguous(), _bias(pw_bias, value.device))
+        on_device(pw_wscale, value.device, torch.float32), bias_on(pw_bias, value.device))
     return out.permute(0, 3, 1, 2)
 
 
@@ -368,7 +380,7 @@ def conv2d_small_cin_quantize_int8(x: Tensor, scale: Tensor, packed: Tensor, bia
     """``quantize_int8(relu(bf16(conv3x3(x)) + bias))`` -> INT8 NHWC ``[B, H, W, Cout]`` (an :class:`Int8Tensor` with
     ``scale``); ``packed`` from :func:`small_cin_prepare`."""
     out = library.conv3x3_small_cin_quantize_int8(x.contiguous(), packed.to(x.device).contiguous(),
-                                                  _bias(bias, x.device), _scalar(scale, x.device))
+                                                  bias_on(bias, x.device), _scalar(scale, x.device))
     return quant.Int8Tensor(out, _same_scale(scale, x.device))
 
 
@@ -390,7 +402,7 @@ def accepts_small_cin(weight: Tensor, bias: Tensor) -> bool:
 
 def bias_relu_quantize_int8(raw: Tensor, bias: Tensor, scale: Tensor) -> quant.Int8Tensor:
     """``quantize_int8(relu(raw + bias))`` of a BF16 NCHW conv output -> INT8 NHWC ``[B, H, W, C]``."""
-    out = library.bias_relu_quantize_int8(raw.contiguous(), _bias(bias, raw.device), _scalar(scale, raw.device))
+    out = library.bias_relu_quantize_int8(raw.contiguous(), bias_on(bias, raw.device), _scalar(scale, raw.device))
     return quant.Int8Tensor(out, _same_scale(scale, raw.device))
 
 

@@ -15,20 +15,12 @@ import torch
 from torch import Tensor
 
 from flashim_amd import library, quant
+from flashim_amd.backends.hip.conv import bias_on, on_device, packed
 from flashim_amd.platforms import is_gfx950
 
 
-def _bias(bias: Tensor | None, device) -> Tensor | None:
-    """FP32 or BF16 ``[N]`` on ``device`` (other dtypes promoted to FP32), or ``None``."""
-    if bias is None:
-        return None
-    if bias.dtype not in (torch.float32, torch.bfloat16):
-        bias = bias.float()
-    return bias.to(device).contiguous()
-
-
 def _a_scale(a_scale: Tensor, device) -> Tensor:
-    return a_scale.to(device=device, dtype=torch.float32).reshape(-1).contiguous()
+    return on_device(a_scale, device, torch.float32).reshape(-1)
 
 
 def int8_linear(a: Tensor, weight: Tensor, a_scale: Tensor, w_scale: Tensor, bias: Tensor | None, *,
@@ -40,8 +32,8 @@ def int8_linear(a: Tensor, weight: Tensor, a_scale: Tensor, w_scale: Tensor, bia
             residual = residual.to(torch.bfloat16)
         if residual.stride(-1) != 1:
             residual = residual.contiguous()
-    return library.int8_linear(a.contiguous(), weight.contiguous(), _a_scale(a_scale, a.device),
-                               w_scale.to(device=a.device, dtype=torch.float32).contiguous(), _bias(bias, a.device),
+    return library.int8_linear(packed(a), packed(weight), _a_scale(a_scale, a.device),
+                               on_device(w_scale, a.device, torch.float32), bias_on(bias, a.device),
                                bool(relu), bool(gelu), residual)
 
 
@@ -51,7 +43,7 @@ def int8_linear_quantize(a: Tensor, weight: Tensor, a_scale: Tensor, w_scale: Te
     with unit column stride and any row stride (``flashim/ops/gemm.py:104-116``). Returns ``out``."""
     library.int8_linear_quantize_(a.contiguous(), weight.contiguous(), _a_scale(a_scale, a.device),
                                   w_scale.to(device=a.device, dtype=torch.float32).contiguous(),
-                                  _bias(bias, a.device), out_scale.to(device=a.device, dtype=torch.float32).reshape(1)
+                                  bias_on(bias, a.device), out_scale.to(device=a.device, dtype=torch.float32).reshape(1)
                                   .contiguous(), out)
     return out
 
@@ -62,7 +54,7 @@ def mxfp8_linear(activation: quant.QuantizedTensor, bias: Tensor | None, weight:
     rows, kpad = a.shape
     out = library.mxfp8_conv2d(
         a.view(1, 1, rows, kpad), activation.scale_exponent.contiguous(), weight.values.contiguous().view(torch.uint8),
-        weight.scale_exponent.contiguous(), _bias(bias, a.device), 1, 1, 1, 1, 0, 0, 1, 1, False, False, None, None)
+        weight.scale_exponent.contiguous(), bias_on(bias, a.device), 1, 1, 1, 1, 0, 0, 1, 1, False, False, None, None)
     return out.view(rows, -1)
 
 
@@ -73,7 +65,7 @@ def mxfp8_scaled_mm(a: Tensor, b_t: Tensor, a_scale: Tensor, b_scale: Tensor, bi
     weight = b_t.t().contiguous()  # [N, K]: a view of the usual transposed weight, no copy
     w_exponent = quant.unswizzle_scales(b_scale, n, k // 32).contiguous()
     return library.mxfp8_scaled_mm(a.contiguous().view(torch.uint8), a_scale.contiguous().view(torch.uint8),
-                                   weight.view(torch.uint8), w_exponent, _bias(bias, a.device))
+                                   weight.view(torch.uint8), w_exponent, bias_on(bias, a.device))
 
 
 MLP_CHANNELS, MLP_HIDDEN = 64, 256  # the fused MLP kernel's shape
@@ -110,17 +102,17 @@ def refiner_mlp(x: Tensor, x_scale: Tensor, w1: Tensor, w1_scale: Tensor, b1: Te
     ``x``: ``[..., 64]``; returns BF16 of the same leading shape."""
     mx = x.dtype == torch.float8_e4m3fn
     lead = x.shape[:-1]
-    a = x.reshape(-1, MLP_CHANNELS).contiguous().view(torch.uint8)
+    a = packed(x.reshape(-1, MLP_CHANNELS))
 
     def scale(t: Tensor) -> Tensor:
-        return t.to(device=a.device, dtype=torch.int8 if mx else torch.float32).contiguous()
+        return on_device(t, a.device, torch.int8 if mx else torch.float32)
 
     res = None
     if residual is not None:
-        res = residual.reshape(-1, MLP_CHANNELS).to(torch.bfloat16).contiguous()
+        res = packed(residual.reshape(-1, MLP_CHANNELS).to(torch.bfloat16))
     out = library.refiner_mlp(
-        1 if mx else 0, 0, a, scale(x_scale), w1.contiguous().view(torch.uint8), scale(w1_scale), _bias(b1, a.device),
-        scale(hidden_scale), w2.contiguous().view(torch.uint8), scale(w2_scale), _bias(b2, a.device), res)
+        1 if mx else 0, 0, a, scale(x_scale), packed(w1), scale(w1_scale), bias_on(b1, a.device), scale(hidden_scale),
+        packed(w2), scale(w2_scale), bias_on(b2, a.device), res)
     return out.view(*lead, MLP_CHANNELS)
 
 

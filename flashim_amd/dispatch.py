@@ -79,8 +79,8 @@ class _Entry:
         """``None`` when this impl applies to the call, else the reason it does not."""
         if not self.device.matches(platform):
             return f"registered for {self.device.type}, call is on {platform.device_type}"
-        missing = [f.value for f in self.requires if not platform.supports(f)]
-        if missing:
+        if not self.requires <= platform.features:
+            missing = [f.value for f in self.requires if not platform.supports(f)]
             return "platform lacks " + ",".join(sorted(missing))
         if check_accepts and self.accepts is not None and not self.accepts(*args[len(args) - weights:]):
             return "accepts() refused the weights"
@@ -238,6 +238,8 @@ class Op:
         if entry.name not in self.calls:
             logger.debug("op %s -> %s", self.name, entry.name)
         self.calls[entry.name] += 1
+        if not _MARKERS and not torch.autograd._profiler_enabled():
+            return entry.fn(*call_args, **kwargs)
         with _range(f"flashim::{self.name}[{entry.name}]"):
             return entry.fn(*call_args, **kwargs)
 

@@ -92,7 +92,8 @@ def _detect(device: torch.device) -> Platform:
 
 
 def platform_for(device: torch.device | str | None = None) -> Platform:
-    device = torch.device(device if device is not None else ("cuda" if torch.cuda.is_available() else "cpu"))
+    if not isinstance(device, torch.device):
+        device = torch.device(device if device is not None else ("cuda" if torch.cuda.is_available() else "cpu"))
     key = (device.type, device.index)
     platform = _PLATFORMS.get(key)
     if platform is None:
@@ -102,7 +103,8 @@ def platform_for(device: torch.device | str | None = None) -> Platform:
 
 @torch.compiler.assume_constant_result  # a process constant per device: keeps dispatch traceable under torch.compile
 def _arch_is_gfx950(device_type: str, index: int | None) -> bool:
-    return platform_for(torch.device(device_type, index)).arch in HIP_ARCHS
+    platform = _PLATFORMS.get((device_type, index)) or platform_for(torch.device(device_type, index))
+    return platform.arch in HIP_ARCHS
 
 
 def is_gfx950(device: torch.device) -> bool:

@@ -134,7 +134,9 @@ def quantize_static(value: Tensor, scale_exponent: Tensor) -> QuantizedTensor:
     _require_gpu(value, "quantize_static")
     _dtype_code(value, "quantize_static")
     padded = padded_channels(value.shape[-1])
-    scale_exponent = scale_exponent.to(device=value.device, dtype=torch.int8).contiguous()
+    if scale_exponent.dtype != torch.int8 or scale_exponent.device != value.device:
+        scale_exponent = scale_exponent.to(device=value.device, dtype=torch.int8)
+    scale_exponent = scale_exponent.contiguous()
     if tuple(scale_exponent.shape) != (padded // BLOCK,):
         raise ValueError(f"Expected scale shape {(padded // BLOCK,)}, got {tuple(scale_exponent.shape)}")
     codes = library.quantize_mxfp8(value, scale_exponent, padded)
@@ -151,7 +153,9 @@ def gelu_quantize_static(value: Tensor, scale_exponent: Tensor, input_bias: Tens
     _require_gpu(value, "gelu_quantize")
     _dtype_code(value, "gelu_quantize")
     padded = padded_channels(value.shape[-1])
-    scale_exponent = scale_exponent.to(device=value.device, dtype=torch.int8).contiguous()
+    if scale_exponent.dtype != torch.int8 or scale_exponent.device != value.device:
+        scale_exponent = scale_exponent.to(device=value.device, dtype=torch.int8)
+    scale_exponent = scale_exponent.contiguous()
     if tuple(scale_exponent.shape) != (padded // BLOCK,):
         raise ValueError(f"Expected scale shape {(padded // BLOCK,)}, got {tuple(scale_exponent.shape)}")
     if input_bias is not None:

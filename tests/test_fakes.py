@@ -128,3 +128,17 @@ def test_gemm_and_block_fakes_match_oracle_shapes():
     raw = torch.randn(1, 16, 5, 6).to(torch.bfloat16)
     assert _fake_run(hc.bias_relu_quantize_int8, raw, torch.randn(16), torch.tensor(0.1)) == \
         _sig(ref.bias_relu_quantize_int8(raw, torch.randn(16), torch.tensor(0.1)))
+
+
+def test_ops_without_a_gpu_kernel_or_derivative_refuse():
+    """The C++ ops have a GPU kernel only, and a tensor that needs a gradient gets an output whose backward raises."""
+    with pytest.raises(NotImplementedError):
+        torch.ops.flashim_amd.quantize_int8(torch.randn(4, 32), torch.ones(()), None)
+    mode = FakeTensorMode()
+    with mode:
+        x = torch.empty(1, 8, 8, 32, device="cuda", dtype=torch.bfloat16).requires_grad_()
+        w, b = torch.empty(25, 32, device="cuda", dtype=torch.bfloat16), torch.empty(32, device="cuda")
+        y = torch.ops.flashim_amd.depthwise5x5(x, w, b, 1, 2, None, None)
+        assert y.requires_grad
+        with pytest.raises(NotImplementedError, match="not implemented"):
+            y.sum().backward()
