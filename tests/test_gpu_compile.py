@@ -77,3 +77,11 @@ def test_compile_depthwise_and_blocks():
     _check(lambda v: ops.depthwise5x5_relu_pointwise_int8(v, dw_w, dw_b, w8, ws, pw_b, s), x)
     pw16 = (torch.randn(c, c, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
     _check(lambda v: ops.depthwise5x5_relu_pointwise(v, dw_w, dw_b, pw16, pw_b), x)
+
+
+def test_backward_through_an_op_raises():
+    x = torch.randn(1, 8, 8, 32, device=DEV).to(torch.bfloat16).requires_grad_()
+    w, b = torch.randn(25, 32, device=DEV).to(torch.bfloat16), torch.randn(32, device=DEV)
+    y = torch.ops.flashim_amd.depthwise5x5(x, w, b, 1, 2, None, None)
+    with pytest.raises(RuntimeError, match="not implemented"):
+        y.float().sum().backward()
