@@ -175,19 +175,44 @@ FIM_HD int8_t quantize_int8_value(float x, float scale) {
   return (int8_t)(int)q;
 }
 
+// x / s as one multiply and two FMAs, for the INT8 rounding: q0 = x inv (inv = RN(1 / s)) clamped to +-256, the remainder
+// x - q0 s (exact where q0 is within 2 ulp of the quotient), and the corrected quotient. Its rounding to an integer,
+// saturated to +-127, equals that of the IEEE division x / s: checked on the host for every BF16 x against 3000 random
+// scales and nice ones (0.04, 0.5, ..., 1e-38, 3e38), infinities included, and for 2e8 FP32 x on and up to 3 ulp around
+// half-integer multiples of random scales. The clamp keeps infinite and huge quotients out of the remainder (they
+// saturate either way); a NaN stays one. Below a scale of 2^-100 the remainder could underflow: there the operands go in
+// scaled by 2^64 (int8_quotient_tiny; values that overflow saturate as well).
+FIM_HD float int8_quotient(float x, float scale, float inv) {
+  float q0 = x * inv;
+#ifdef __HIP_DEVICE_COMPILE__
+  q0 = __builtin_amdgcn_fmed3f(q0, -256.0f, 256.0f);
+#else
+  q0 = q0 < -256.0f ? -256.0f : q0 > 256.0f ? 256.0f : q0;
+#endif
+  return fmaf(fmaf(-q0, scale, x), inv, q0);
+}
+
+FIM_HD bool int8_scale_is_tiny(float scale) { return scale < 0x1p-100f; }
+
+FIM_HD float int8_quotient_tiny(float x, float scale, float inv) {
+  return int8_quotient(x * 0x1p64f, scale * 0x1p64f, inv * 0x1p-64f);
+}
+
 #ifdef __HIPCC__
-// quantize_int8_value with the division replaced by a multiply by inv = 1 / scale (correctly rounded), falling back
-// to the IEEE division only where it can matter: x * inv is within a few ulps of the exact quotient, so both round to
-// the same integer unless the quotient sits within 2^-15 of a half-integer; beyond |q| = 127 both saturate. The
+// quantize_int8_value with the division replaced by a multiply by inv = 1 / scale (correctly rounded), and by the
+// corrected quotient (int8_quotient) where that can matter: x * inv is within a few ulps of the exact quotient, so both
+// round to the same integer unless the quotient sits within 2^-15 of a half-integer; beyond |q| = 127 both saturate. The
 // rounding is one FMA with M = 1.5 * 2^23: fma(x, inv, M) rounds x * inv + M once, to the nearest integer (ties to
 // even) on the grid of unit spacing where M sits, so its low mantissa bits hold rint(x * inv) and its low byte is the
 // INT8 code in two's complement; r = f - M (exact) is the rounded quotient and fma(x, inv, -r) the exact residual, and
-// |residual| >= 0.5 - 2^-15 marks a near-tie. The fallback sits behind one wave-uniform branch for all N values (taken
-// when any lane is near a tie), so it neither runs per element nor splits the code that produces the inputs. The
+// |residual| >= 0.5 - 2^-15 marks a near-tie. The correction sits behind one wave-uniform branch for all N values (taken
+// when any lane is near a tie), so it does not split the code that produces the inputs, and has no branch of its own:
+// BF16 values over a scale such as 0.04 or 0.5 meet exact ties in nearly every batch (an IEEE division behind a branch
+// per value there made up 40% of the VGG stem's time). The
 // saturation is one v_med3_f32 between M - 127 and M + 127 (LO = 0 folds a preceding ReLU in: relu then quantize
 // equals clamping the rounded quotient at 0), so no conversion to an integer is needed: q[i] holds the clamped value's
 // bit pattern, whose low byte is the code (callers keep that byte). 5 VALU operations per value (FMA, subtraction,
-// residual FMA, running maximum, med3), none on the scalar unit. Checked on the host
+// residual FMA, running maximum, med3), 5 more with the correction, none on the scalar unit. Checked on the host
 // against round(x / s) on 20M cases including exact ties and their neighbours, with and without the ReLU, and on the
 // GPU byte for byte against the torch references of every INT8 producer.
 template <int N, int LO = -127>
@@ -204,9 +229,13 @@ __device__ __forceinline__ void quantize_int8_fast_n(const float (&x)[N], float 
     worst = fmaxf(worst, fabsf(fmaf(x[i], inv, -(f[i] - M))));
   }
   if (__builtin_amdgcn_ballot_w64(worst >= NEAR) != 0) {
+    if (!int8_scale_is_tiny(scale)) {  // uniform
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-      if (fabsf(fmaf(x[i], inv, -(f[i] - M))) >= NEAR) f[i] = __builtin_rintf(__fdiv_rn(x[i], scale)) + M;
+      for (int i = 0; i < N; ++i) f[i] = int8_quotient(x[i], scale, inv) + M;
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) f[i] = int8_quotient_tiny(x[i], scale, inv) + M;
+    }
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) q[i] = __builtin_bit_cast(int, __builtin_amdgcn_fmed3f(f[i], M + (float)LO, M + 127.0f));

@@ -29,6 +29,15 @@ void fim_host_bf16(const float* x, int64_t n, uint16_t* out) {
   for (int64_t i = 0; i < n; ++i) out[i] = fim::f32_to_bf16(x[i]);
 }
 
+// the corrected quotient's codes, as the device quantizer's near-tie path computes them
+void fim_host_int8_quotient(const float* x, int64_t n, float scale, int8_t* out) {
+  volatile float inv = 1.0f / scale;
+  for (int64_t i = 0; i < n; ++i) {
+    const float q = rintf(fim::int8_scale_is_tiny(scale) ? fim::int8_quotient_tiny(x[i], scale, inv)
+                                                         : fim::int8_quotient(x[i], scale, inv));
+    out[i] = (int8_t)(int)(q > 127.0f ? 127.0f : q < -127.0f ? -127.0f : q);
+  }
+}
 void fim_host_quantize_int8(const float* x, int64_t n, float scale, int8_t* out) {
   for (int64_t i = 0; i < n; ++i) out[i] = fim::quantize_int8_value(x[i], scale);
 }

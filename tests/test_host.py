@@ -174,6 +174,21 @@ def test_host_bf16_and_int8_rounding_match_torch():
     assert np.array_equal(got, ref.quantize_int8_static(y, torch.tensor(0.37)).numpy())
 
 
+@pytest.mark.parametrize("scale", [0.04, 0.05, 0.5, 1.0, 0.017, 3.3e-5, 1.1920929e-07, 1e-38, 3e38])
+def test_host_int8_quotient_rounds_as_the_division(scale):
+    """The near-tie path of the device quantizer (a multiply and two FMAs) against rint of the IEEE quotient: every
+    finite and infinite BF16 value, and FP32 values on and next to half-integer multiples of the scale."""
+    h = _lib.load_host()
+    s = torch.tensor(scale)
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).float()
+    ties = (torch.arange(-130, 130).double() + 0.5) * s.double()
+    near = torch.stack([ties.float(), torch.nextafter(ties.float(), torch.tensor(torch.inf)),
+                        torch.nextafter(ties.float(), torch.tensor(-torch.inf))]).flatten()
+    x = torch.cat([x[~x.isnan()], near[near.isfinite()]])
+    got = _call(h.fim_host_int8_quotient, x.numpy(), np.int8, ctypes.c_float(scale))
+    assert np.array_equal(got, (x / s).round().clamp(-127, 127).to(torch.int8).numpy())
+
+
 # -- the dispatcher ----------------------------------------------------------------------------------------------
 
 
