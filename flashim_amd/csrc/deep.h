@@ -11,7 +11,7 @@
 // takes 12 steps of a 3 x 3 filter instead of 18), and INT8 inputs and outputs of any multiple of 4 channels are taken.
 // Measured (MI355X): a 160 x 256 step 1570 clocks for 1280 of MFMA issue, at the 1.75 to 1.9 GHz that the matrix cores'
 // power draw leaves; prologue 3.3 us, epilogue 3 to 6 us. INT8 512 -> 512 3 x 3 at 112 x 150 75 -> 49 us, MXFP8 256 -> 256
-// at 224 x 300 67 -> 50 us, INT8 196 -> 128 at 448 x 600 970 -> 118 us (it ran on byte loads).
+// at 224 x 300 67 -> 50 us, INT8 196 -> 128 at 448 x 600 970 -> 108 us (it ran on byte loads).
 #pragma once
 
 #include "deep_plan.h"
@@ -33,8 +33,9 @@ __device__ __forceinline__ int div_magic(int n, uint32_t mul, int shift) {
   return shift < 0 ? n : (int)(__umulhi((uint32_t)n, mul) >> shift);
 }
 
-template <int KIND, int OUT, int WN, int MBW, bool RAG>
-__global__ __launch_bounds__(256, 1) void conv_deep_kernel(const DeepArgs d) {
+// TWO: two workgroups per CU (128 x 128 tiles in two stages), which cover each other's prologues, epilogues and waits.
+template <int KIND, int OUT, int WN, int MBW, bool RAG, bool TWO = false>
+__global__ __launch_bounds__(256, TWO ? 2 : 1) void conv_deep_kernel(const DeepArgs d) {
   constexpr int WM = 4 / WN, BR = DEEP_BR;
   constexpr int BM = WM * MBW * BR, BN = WN * 64;
   // a stage: the weight rows, then the activation rows, in 8-row chunks (one wave-wide 16-byte-per-lane load each);
@@ -42,7 +43,7 @@ __global__ __launch_bounds__(256, 1) void conv_deep_kernel(const DeepArgs d) {
   // four, wavefronts 2 and 3 load wavefront 0's and 1's again)
   constexpr int ACH = BM / 8, NW = BN / 32, NA = (ACH + 3) / 4, CHUNKS = NW + NA;
   constexpr int STAGE = (BM + BN) * KC;
-  constexpr int NST = deep_stages(KIND == KIND_MX, BM, BN);
+  constexpr int NST = TWO ? 2 : deep_stages(KIND == KIND_MX, BM, BN);
   // The software pipeline over a step's 32-row blocks: a block's operands are read during the block before it, and the
   // last L blocks' MFMAs run after the barrier that ends the step, while the next step's first operands are read. The
   // reads and the next stage's loads are placed one by one between the MFMAs (a load issued behind another waits for

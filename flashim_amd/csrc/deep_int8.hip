@@ -15,7 +15,9 @@ static int launch_out(const ConvArgs& a, DeepPlan p, hipStream_t stream) {
     }
   } else if (p.wn == 2) {
     switch (p.mbw) {
-      case 2: return launch_deep_tile<KIND_INT8, OUT, 2, 2, RAG>(a, stream);
+      case 2:
+        return p.two ? launch_deep_tile<KIND_INT8, OUT, 2, 2, RAG, true>(a, stream)
+                     : launch_deep_tile<KIND_INT8, OUT, 2, 2, RAG>(a, stream);
       case 3: return launch_deep_tile<KIND_INT8, OUT, 2, 3, RAG>(a, stream);
       case 4: return launch_deep_tile<KIND_INT8, OUT, 2, 4, RAG>(a, stream);
       case 5: return launch_deep_tile<KIND_INT8, OUT, 2, 5, RAG>(a, stream);

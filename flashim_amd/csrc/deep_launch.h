@@ -32,11 +32,11 @@ inline DeepArgs deep_args(const ConvArgs& a, int bm, int bn) {
   return d;
 }
 
-template <int KIND, int OUT, int WN, int MBW, bool RAG>
+template <int KIND, int OUT, int WN, int MBW, bool RAG, bool TWO = false>
 inline int launch_deep_tile(const ConvArgs& a, hipStream_t stream) {
   const DeepArgs d = deep_args(a, (4 / WN) * MBW * DEEP_BR, WN * 64);
   const dim3 grid((unsigned)(cdiv((int64_t)d.c.n_tiles * d.c.m_tiles, 8) * 8));
-  conv_deep_kernel<KIND, OUT, WN, MBW, RAG><<<grid, dim3(256), 0, stream>>>(d);
+  conv_deep_kernel<KIND, OUT, WN, MBW, RAG, TWO><<<grid, dim3(256), 0, stream>>>(d);
   return launch_status();
 }
 

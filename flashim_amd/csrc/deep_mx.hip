@@ -15,7 +15,9 @@ static int launch_out(const ConvArgs& a, DeepPlan p, hipStream_t stream) {
     }
   } else if (p.wn == 2) {
     switch (p.mbw) {
-      case 2: return launch_deep_tile<KIND_MX, OUT, 2, 2, false>(a, stream);
+      case 2:
+        return p.two ? launch_deep_tile<KIND_MX, OUT, 2, 2, false, true>(a, stream)
+                     : launch_deep_tile<KIND_MX, OUT, 2, 2, false>(a, stream);
       case 3: return launch_deep_tile<KIND_MX, OUT, 2, 3, false>(a, stream);
       case 4: return launch_deep_tile<KIND_MX, OUT, 2, 4, false>(a, stream);
       case 5: return launch_deep_tile<KIND_MX, OUT, 2, 5, false>(a, stream);

@@ -14,7 +14,7 @@ constexpr int DEEP_CBLOCKS = 256;
 // wavefront; rag: Cin or Cout not a multiple of 16. wn 0: the deep kernel does not take the launch.
 struct DeepPlan {
   int wn, mbw;
-  bool rag;
+  bool rag, two;  // two: 128 x 128 tiles, two workgroups per CU
 };
 
 int launch_deep_int8(const ConvArgs& a, DeepPlan p, hipStream_t stream);

@@ -20,9 +20,9 @@ static double step_clocks(int wn, int bm, int bn, bool three_stages) {
 // 128-byte K step 1.65 us a round of 512 tiles (0.45 to 1.5 us for launches of fewer than 256, which run as 64 x 64
 // tiles; 13.5 us a round, at least 6, where Cin is no multiple of 16: byte loads). Measured, deep
 // against 128-row: INT8 512 -> 512 at 112 x 150 49 / 75 us, MXFP8 256 -> 256 at 224 x 300 50 / 67 us, INT8 196 -> 128 at
-// 448 x 600 118 / 970 us; one-step 1 x 1 layers the other way round (64 -> 256 at 233 x 286 23 / 21 us).
+// 448 x 600 108 / 970 us; one-step 1 x 1 layers the other way round (64 -> 256 at 233 x 286 23 / 21 us).
 DeepPlan deep_plan(const ConvArgs& a, int kind) {
-  const DeepPlan none = {0, 0, false};
+  const DeepPlan none = {0, 0, false, false};
   const bool mx = kind == KIND_MX;
   if (a.x_swz != nullptr || a.pool_out != nullptr || a.a_scale_rows != nullptr || a.gelu || a.Cout <= 64) return none;
   if (a.out_mode == (mx ? OUT_INT8 : OUT_E4M3)) return none;
@@ -54,13 +54,19 @@ DeepPlan deep_plan(const ConvArgs& a, int kind) {
       const int nst = deep_stages(mx, bm, bn);
       const int64_t rounds = cdiv(cdiv((int64_t)a.M, bm) * cdiv((int64_t)a.Cout, bn), cus);
       const int64_t nk = cdiv(cdiv((int64_t)taps * cdiv((int64_t)a.Cin, 16), 8), nst) * nst;
-      const double epilogue = bm * bn * (a.out_mode == OUT_INT8 ? 0.33 : 0.19);
-      const double t = 2 * US + rounds * (nk * step_clocks(wn, bm, bn, nst == 3) + 7500 + epilogue);
+      const double epilogue = bm * bn * ((a.out_mode == OUT_INT8 ? 0.33 : 0.19) + (rag ? 0.12 : 0));
+      const double mask = rag_in ? 300.0 * bm / 256 : 0;
+      const double t = 2 * US + rounds * (nk * (step_clocks(wn, bm, bn, nst == 3) + mask) + 7500 + epilogue);
       if (t < best) {
         best = t;
-        p = {wn, mbw, rag};
+        p = {wn, mbw, rag, false};
       }
     }
+  // two 128 x 128 workgroups per CU: a pair's step is slower than a large tile's, but the round's prologue and epilogue
+  // are half covered, which pays where several rounds of few steps run (INT8 196 -> 320 1 x 1 at 2 x 111 x 177 27 -> 21 us)
+  const int64_t pairs = cdiv(cdiv((int64_t)a.M, 128) * cdiv((int64_t)a.Cout, 128), 2 * cus);
+  const int64_t nk2 = cdiv(cdiv((int64_t)taps * cdiv((int64_t)a.Cin, 16), 8), 2) * 2;
+  if (2 * US + pairs * (nk2 * (rag_in ? 1850 : 1700) + 11500) < best) p = {2, 2, rag, true};
   return p;
 }
 

@@ -80,3 +80,11 @@ def test_mxfp8_deep_conv_matches_general_path(shape, out_e4m3, residual):
     # E4M3: a code moves by one step (2^-3 of its value) where its BF16 value moved across a rounding boundary: about one
     # in 2^5 of the moved BF16 values, themselves rarer than one in 10^3, so the same bar holds
     assert ((got - want).norm() / want.norm()).item() <= 1e-3
+
+
+@pytest.mark.parametrize("shape", [(2, 111, 177, 196, 320, 1, 1, 0, 1), (2, 208, 326, 68, 160, 3, 1, 1, 1),
+                                   (2, 392, 214, 68, 224, 1, 1, 0, 1)])
+@pytest.mark.parametrize("out_int8", [False, True])
+def test_int8_deep_conv_two_workgroups_per_cu(shape, out_int8):
+    """Several rounds of few K steps: 128 x 128 tiles, two workgroups per CU."""
+    test_int8_deep_conv_matches_general_path(shape, out_int8, False)
