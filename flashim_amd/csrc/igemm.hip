@@ -1022,8 +1022,8 @@ __global__ __launch_bounds__(512, 1) void conv_patch_kernel(const ConvArgs a) {
 // 18.98 us; 12 x 16 tiles, 884 of them, at most 4 for 3.45, 19.5 us; 4 x 16, 19.8 us).
 constexpr int PATCH_TH = 8, PATCH_TW = 16;
 
-static int64_t patch_grid(int64_t tiles, int64_t n_tiles) {
-  // a multiple of 8 (XCDs) and of the channel-block count (each workgroup keeps one), at most one per CU
+static int64_t patch_grid(int64_t tiles, int64_t n_tiles, int64_t per_cu = 1) {
+  // a multiple of 8 (XCDs) and of the channel-block count (each workgroup keeps one), at most per_cu per CU
   int64_t x = 8, y = n_tiles;
   while (y != 0) {
     const int64_t r = x % y;
@@ -1031,7 +1031,7 @@ static int64_t patch_grid(int64_t tiles, int64_t n_tiles) {
     y = r;
   }
   const int64_t unit = 8 * n_tiles / x;
-  const int64_t cap = std::max<int64_t>(unit, device_cus() / unit * unit);
+  const int64_t cap = std::max<int64_t>(unit, per_cu * device_cus() / unit * unit);
   return std::min<int64_t>(cdiv(tiles, unit) * unit, cap);
 }
 
@@ -1062,15 +1062,25 @@ static int launch_patch(ConvArgs a, hipStream_t stream) {
 // ---- Pointwise, register operands --------------------------------------------------------------------------------
 // Pointwise (1 x 1, stride 1) convolutions, a GEMM over pixels, with Cin % 128 == 0, Cin <= 512 or 1024, and Cout >=
 // 128, where the epilogue (GELU above all) or the HBM traffic (big-K contracts) outweighs the MFMAs. Persistent
-// workgroups of 8 wavefronts, one per CU, keep the weights of 128 output channels in LDS (128 x Cin bytes, read-only
-// after the prologue); every wavefront then works alone, with no barrier: it loads its tile's 32 pixel rows of
-// activations straight into MFMA operand registers (up to 4 K steps at a time), runs 2 x 8 blocks of 16 x 16 against
-// the LDS weights, and writes its epilogue through a private LDS staging area in whole lines. Two wavefronts per SIMD drift apart, so one's loads
-// and MFMAs run while the other's epilogue keeps the VALU busy.
+// workgroups keep the weights of 128 output channels in LDS (128 x Cin bytes, read-only after the prologue); every
+// wavefront then works alone, with no barrier: it loads its tile's 32 pixel rows of activations straight into MFMA
+// operand registers (up to 4 K steps at a time), runs 2 x 8 blocks of 16 x 16 against the LDS weights, and writes its
+// epilogue through a private LDS staging area in whole lines. The two or three wavefronts of a SIMD drift apart, so
+// one's loads and MFMAs run while another's epilogue keeps the VALU busy.
 // XS = 1: MXFP8 activations with per-row E8M0 scales in the 128x4 swizzled layout (mxfp8_scaled_mm's dynamic
 // quantization), read per tile with the rows; XS = 0: per-channel-block exponents.
+// Quantized outputs of at most 256 input channels are bound by the epilogue's VALU chains (GELU, the codes), not by
+// memory, and fit 168 VGPRs: workgroups of 4 wavefronts, three per CU, put 3 wavefronts on a SIMD instead of 2 (128 ->
+// 512 channels over 320000 pixels with GELU: INT8 155 -> 143 us, MXFP8 113 -> 105; 256 -> 1024 over 80000: 86 -> 84
+// and 67 -> 66). BF16 outputs spill there and are bound by their stores (128 channels, 320000 pixels: INT8 25 -> 28 us;
+// 256 channels, 80000 pixels: MXFP8 69 -> 84), so they keep 8 wavefronts, one workgroup per CU, as do the deeper K,
+// whose weights fill the LDS.
+constexpr int pw_waves(int ks, int out) { return ks <= 2 && out != OUT_BF16 ? 4 : 8; }
+constexpr int pw_per_simd(int ks, int out) { return ks <= 2 && out != OUT_BF16 ? 3 : 2; }
+
 template <int KIND, int OUT, int KS, int XS = 0>
-__global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
+__global__ __launch_bounds__(64 * pw_waves(KS, OUT), pw_per_simd(KS, OUT)) void conv_pw_kernel(const ConvArgs a) {
+  constexpr int NW = pw_waves(KS, OUT);                   // wavefronts
   constexpr int BN = 128, MB = 2, NB = 8, TMW = MB * 16;  // a wavefront's tile: 32 pixels x 128 channels
   constexpr int WTS_BYTES = KS * BN * KC;                // [K step][channel][128 B]
   constexpr int XEXP_BYTES = (KS * 4 + 15) / 16 * 16;    // the activations' MX exponent bytes (XS = 0)
@@ -1086,7 +1096,7 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
   constexpr int RB = (HS ? BN / 2 : BN) * ESZ, LPP = RB / 16, PPC = 64 / LPP;
   constexpr int SCH = 16 / PPC;  // 1 KB stores per 16-pixel round
   static_assert(SCH * PPC == 16, "whole stores per round");
-  constexpr int STAGE_BYTES = 8 * 16 * RB;
+  constexpr int STAGE_BYTES = NW * 16 * RB;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[WTS_BYTES + STAGE_BYTES + WEXP_BYTES + 3 * BN * 4 + XEXP_BYTES];
   uint8_t* const wts = smem;
   uint8_t* const stage = wts + WTS_BYTES;
@@ -1101,9 +1111,9 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4;
 
-  // tiles: 8 x 32 pixels x 128 channels, wavefront w taking pixels [32 w, +32); XCD-aware deal as in the patch kernel,
+  // tiles: NW x 32 pixels x 128 channels, wavefront w taking pixels [32 w, +32); XCD-aware deal as in the patch kernel,
   // the workgroup keeping one channel block
-  const int m_tiles = (a.M + 8 * TMW - 1) / (8 * TMW);
+  const int m_tiles = (a.M + NW * TMW - 1) / (NW * TMW);
   const int total = a.n_tiles * m_tiles;
   const int stride = gridDim.x;
   const int per_xcd = stride >> 3;
@@ -1115,8 +1125,8 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
   const int w_nrec = __builtin_amdgcn_readfirstlane(a.Cout * a.Cin);
   constexpr uint32_t OOB = 0x80000000u;
 #pragma unroll
-  for (int i = 0; i < KS * BN / 64; ++i) {  // weights: chunk k (8 channels x 128 bytes of one K step) = wave + 8 i
-    const int k = wave + 8 * i;
+  for (int i = 0; i < KS * BN / 8 / NW; ++i) {  // weights: chunk k (8 channels x 128 bytes of one K step) = wave + NW i
+    const int k = wave + NW * i;
     const int ks = k / (BN / 8), r = 8 * (k % (BN / 8)) + (lane >> 3);
     const int seg = (lane & 7) ^ patch_swz(r);
     const uint32_t off = n0 + r < a.Cout ? (uint32_t)((n0 + r) * a.Cin + ks * KC + seg * 16) : OOB;
@@ -1136,17 +1146,17 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
     ep_osc[tid] = (OUT == OUT_E4M3 && nok) ? exp2_int((int)a.out_expo[n >> 5]) : 1.0f;
   }
   if constexpr (KIND == KIND_MX) {
-    constexpr int WEXP_N = BN * KS * 4, WEXP_PASSES = (WEXP_N + 511) / 512;
+    constexpr int WEXP_N = BN * KS * 4, WEXP_PASSES = (WEXP_N + 64 * NW - 1) / (64 * NW);
     const int64_t wexp_valid = ((int64_t)a.Cout - n0) * (KS * 4);
     int e[WEXP_PASSES];
 #pragma unroll
     for (int i = 0; i < WEXP_PASSES; ++i) {
-      const int idx = tid + 512 * i;
+      const int idx = tid + 64 * NW * i;
       e[i] = idx < WEXP_N && idx < wexp_valid ? w_scale_byte(a, a.w_expo[(int64_t)n0 * (KS * 4) + idx]) : 127;
     }
 #pragma unroll
     for (int i = 0; i < WEXP_PASSES; ++i)
-      if (tid + 512 * i < WEXP_N) wexp_s[tid + 512 * i] = (uint8_t)e[i];
+      if (tid + 64 * NW * i < WEXP_N) wexp_s[tid + 64 * NW * i] = (uint8_t)e[i];
     if (XS == 0 && tid < KS * 4) xexp_s[tid] = (uint8_t)((int)a.x_expo[tid] + 127);
   }
 
@@ -1155,7 +1165,7 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
   const __amdgpu_buffer_rsrc_t xr =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.x), (short)0, x_nrec, 0x00020000);
   auto load_x = [&](int t, int kb, v8i (&xa)[MB][KH], int (&sr)[MB][KH]) __attribute__((always_inline)) {
-    const int m0 = (t / a.n_tiles) * (8 * TMW) + wave * TMW;
+    const int m0 = (t / a.n_tiles) * (NW * TMW) + wave * TMW;
 #pragma unroll
     for (int j = 0; j < MB; ++j) {
       const int m = m0 + j * 16 + (lane & 15);
@@ -1180,15 +1190,12 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
     }
   };
 
-  int wo[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const int r = i * 16 + (lane & 15);
-    wo[i] = r * KC + ((g ^ patch_swz(r)) << 4);
-  }
-  auto read_w = [&](int ofs) __attribute__((always_inline)) {
-    const v4i lo = *reinterpret_cast<const v4i*>(smem + ofs);
-    const v4i hi = *reinterpret_cast<const v4i*>(smem + (ofs ^ 64));
+  // weight operands: the swizzle repeats every 16 rows, so a K half's rows of all blocks and steps lie at constant
+  // distances from one address
+  const int wo = (lane & 15) * KC + ((g ^ patch_swz(lane & 15)) << 4);
+  auto read_w = [&](const int (&wq)[2], int ofs) __attribute__((always_inline)) {
+    const v4i lo = *reinterpret_cast<const v4i*>(smem + wq[0] + ofs);
+    const v4i hi = *reinterpret_cast<const v4i*>(smem + wq[1] + ofs);
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
@@ -1220,12 +1227,8 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
 
   // one tile: its operand loads are waited for right away; the other wavefront on the SIMD runs meanwhile
   auto run_tile = [&](int t) __attribute__((always_inline)) {
-    int wq[NB];  // weight offsets made opaque per tile (else all K steps' weight operands are hoisted)
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      wq[i] = wo[i];
-      asm volatile("" : "+v"(wq[i]));
-    }
+    int wq[2] = {wo, wo ^ 64};  // made opaque per tile (else all K steps' weight operands are hoisted)
+    asm volatile("" : "+v"(wq[0]), "+v"(wq[1]));
     v4i acc_i[NB][MB];
     v4f acc_f[NB][MB];
 #pragma unroll
@@ -1241,14 +1244,14 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
       int sr[MB][KH];  // per-row scales (XS = 1)
       load_x(t, kb, xc, sr);
       v8i wc[2];
-      wc[0] = read_w(wq[0] + kb * (BN * KC));
+      wc[0] = read_w(wq, kb * (BN * KC));
 #pragma unroll
       for (int k = 0; k < KH; ++k)
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
           const int ks = kb + k;
           const int nx = k * NB + i + 1;  // the next weight block of this phase, read while this one's MFMAs run
-          if (nx < KH * NB) wc[nx & 1] = read_w(wq[nx % NB] + (kb + nx / NB) * (BN * KC));
+          if (nx < KH * NB) wc[nx & 1] = read_w(wq, (kb + nx / NB) * (BN * KC) + nx % NB * (16 * KC));
           const v8i& w = wc[(k * NB + i) & 1];
 #pragma unroll
           for (int j = 0; j < MB; ++j) {
@@ -1277,7 +1280,7 @@ __global__ __launch_bounds__(512, 1) void conv_pw_kernel(const ConvArgs a) {
           asm volatile("" : "+v"(acc_f[i][j]));
       }
     // epilogue: 16 pixels per round, staged in this wavefront's LDS area and written in whole lines
-    const int m0 = (t / a.n_tiles) * (8 * TMW) + wave * TMW;
+    const int m0 = (t / a.n_tiles) * (NW * TMW) + wave * TMW;
     const int sl = lane % LPP;
     // the staged rows out in whole lines: 16 pixels x RB bytes, from channel n0 + nh on
     auto write_stage = [&](int r, int nh) __attribute__((always_inline)) {
@@ -1349,12 +1352,13 @@ static int pw_ks(const ConvArgs& a, int lw, bool fast_ok) {
 
 template <int KIND, int OUT, int XS>
 static void launch_pw_ks(const ConvArgs& a, int ks, dim3 grid, hipStream_t stream) {
+  const dim3 block(64 * pw_waves(ks, OUT));
   switch (ks) {
-    case 1: conv_pw_kernel<KIND, OUT, 1, XS><<<grid, dim3(512), 0, stream>>>(a); break;
-    case 2: conv_pw_kernel<KIND, OUT, 2, XS><<<grid, dim3(512), 0, stream>>>(a); break;
-    case 3: conv_pw_kernel<KIND, OUT, 3, XS><<<grid, dim3(512), 0, stream>>>(a); break;
-    case 4: conv_pw_kernel<KIND, OUT, 4, XS><<<grid, dim3(512), 0, stream>>>(a); break;
-    default: conv_pw_kernel<KIND, OUT, 8, XS><<<grid, dim3(512), 0, stream>>>(a); break;
+    case 1: conv_pw_kernel<KIND, OUT, 1, XS><<<grid, block, 0, stream>>>(a); break;
+    case 2: conv_pw_kernel<KIND, OUT, 2, XS><<<grid, block, 0, stream>>>(a); break;
+    case 3: conv_pw_kernel<KIND, OUT, 3, XS><<<grid, block, 0, stream>>>(a); break;
+    case 4: conv_pw_kernel<KIND, OUT, 4, XS><<<grid, block, 0, stream>>>(a); break;
+    default: conv_pw_kernel<KIND, OUT, 8, XS><<<grid, block, 0, stream>>>(a); break;
   }
 }
 
@@ -1372,8 +1376,9 @@ static void launch_pw_out(const ConvArgs& a, int ks, dim3 grid, hipStream_t stre
 template <int KIND>
 static int launch_pw(ConvArgs a, int ks, hipStream_t stream) {
   a.n_tiles = (int)cdiv(a.Cout, 128);
-  const int64_t tiles = cdiv((int64_t)a.M, 256) * a.n_tiles;
-  const dim3 grid((unsigned)patch_grid(tiles, a.n_tiles));
+  const int waves = pw_waves(ks, a.out_mode);
+  const int64_t tiles = cdiv((int64_t)a.M, 32 * waves) * a.n_tiles;
+  const dim3 grid((unsigned)patch_grid(tiles, a.n_tiles, 4 * pw_per_simd(ks, a.out_mode) / waves));
   constexpr int QOUT = KIND == KIND_INT8 ? OUT_INT8 : OUT_E4M3;
   if (a.out_mode == OUT_BF16)
     launch_pw_out<KIND, OUT_BF16>(a, ks, grid, stream);

@@ -578,3 +578,30 @@ def test_mxfp8_conv2d_pointwise_tiles(case):
         got_q = hip(*args, *PW_GEO, out_exponent=oe.to(DEV))
         assert torch.equal(got_q.view(torch.uint8), ops.quantize_mxfp8(hip(*args, *PW_GEO), oe.to(DEV)).values
                            .view(torch.uint8)), name
+
+
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("kind", ["int8", "mxfp8"])
+@pytest.mark.parametrize("pixels, cin, cout", [(131073, 128, 128), (131199, 256, 128), (65537, 128, 160),
+                                               (65663, 256, 192)])
+def test_pointwise_quantized_outputs(pixels, cin, cout, kind, gelu):
+    """The pointwise kernel's quantized outputs (4 wavefronts to a workgroup) are the codes of its own BF16 outputs (8
+    wavefronts), one pixel and one pixel short of a whole tile past the last 128: both sum the same K blocks in order."""
+    torch.manual_seed(pixels + cin)
+    if kind == "int8":
+        args = _dev(*_int8_inputs(cin, cout, 1, 1, True, shape=(1, 1, pixels)))
+        hip = ops.int8_conv2d.get("hip")
+        scale = torch.tensor(0.09, device=DEV)
+        got = hip(*args, *PW_GEO, gelu=gelu, out_scale=scale)
+        want = ops.quantize_int8(hip(*args, *PW_GEO, gelu=gelu), scale).values
+    else:
+        x = (torch.randn(1, 1, pixels, cin) * 3).to(torch.float8_e4m3fn)
+        ce = torch.randint(-6, 3, (cin // 32,), dtype=torch.int8)
+        w = (torch.randn(cout, cin) * 2).to(torch.float8_e4m3fn)
+        we = torch.randint(-10, -4, (cout, cin // 32), dtype=torch.int8)
+        args = _dev(x, ce, w, we, torch.randn(cout).to(torch.bfloat16))
+        hip = ops.mxfp8_conv2d.get("hip")
+        exponent = torch.randint(-3, 2, (cout // 32,), dtype=torch.int8).to(DEV)
+        got = hip(*args, *PW_GEO, gelu=gelu, out_exponent=exponent)
+        want = ops.quantize_mxfp8(hip(*args, *PW_GEO, gelu=gelu), exponent).values
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
