@@ -180,8 +180,8 @@ FIM_HD int8_t quantize_int8_value(float x, float scale) {
 // saturated to +-127, equals that of the IEEE division x / s: checked on the host for every BF16 x against 3000 random
 // scales and nice ones (0.04, 0.5, ..., 1e-38, 3e38), infinities included, and for 2e8 FP32 x on and up to 3 ulp around
 // half-integer multiples of random scales. The clamp keeps infinite and huge quotients out of the remainder (they
-// saturate either way); a NaN stays one. Below a scale of 2^-100 the remainder could underflow: there the operands go in
-// scaled by 2^64 (int8_quotient_tiny; values that overflow saturate as well).
+// saturate either way); a NaN stays one. Where the scale's magnitude is below 2^-100 the remainder could underflow: there
+// the operands go in scaled by 2^64 (int8_quotient_tiny; values that overflow saturate as well).
 FIM_HD float int8_quotient(float x, float scale, float inv) {
   float q0 = x * inv;
 #ifdef __HIP_DEVICE_COMPILE__
@@ -192,7 +192,7 @@ FIM_HD float int8_quotient(float x, float scale, float inv) {
   return fmaf(fmaf(-q0, scale, x), inv, q0);
 }
 
-FIM_HD bool int8_scale_is_tiny(float scale) { return scale < 0x1p-100f; }
+FIM_HD bool int8_scale_is_tiny(float scale) { return fabsf(scale) < 0x1p-100f; }
 
 FIM_HD float int8_quotient_tiny(float x, float scale, float inv) {
   return int8_quotient(x * 0x1p64f, scale * 0x1p64f, inv * 0x1p-64f);

@@ -174,7 +174,7 @@ def test_host_bf16_and_int8_rounding_match_torch():
     assert np.array_equal(got, ref.quantize_int8_static(y, torch.tensor(0.37)).numpy())
 
 
-@pytest.mark.parametrize("scale", [0.04, 0.05, 0.5, 1.0, 0.017, 3.3e-5, 1.1920929e-07, 1e-38, 3e38])
+@pytest.mark.parametrize("scale", [0.04, 0.05, 0.5, 1.0, 0.017, 3.3e-5, 1.1920929e-07, 1e-38, 3e38, -0.04, -4e19, -1e-38])
 def test_host_int8_quotient_rounds_as_the_division(scale):
     """The near-tie path of the device quantizer (a multiply and two FMAs) against rint of the IEEE quotient: every
     finite and infinite BF16 value, and FP32 values on and next to half-integer multiples of the scale."""
