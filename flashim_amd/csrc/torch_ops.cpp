@@ -50,6 +50,11 @@ void check(int code, const What&... what) {
   TORCH_CHECK(false, what..., " launch failed (code ", code, ")");
 }
 
+// size() and stride() of the leading dimensions would read an input of more dimensions as one of fewer
+void check_dims(const Tensor& t, int64_t dims, const char* what) {
+  TORCH_CHECK_VALUE(t.dim() == dims, what, ": expected ", dims, " dimensions, got shape ", t.sizes());
+}
+
 Tensor empty(at::IntArrayRef sizes, const Tensor& like, at::ScalarType dtype) {
   return at::empty(sizes, like.options().dtype(dtype).requires_grad(false).memory_format(std::nullopt));
 }
@@ -124,6 +129,7 @@ Tensor swizzled_scales(int64_t rows, int64_t groups, const Tensor& like) {
 }
 
 std::tuple<Tensor, Tensor> quantize_mxfp8_dynamic(const Tensor& value_in, bool swizzled) {
+  check_dims(value_in, 2, "quantize_mxfp8_dynamic");
   const c10::DeviceGuard guard(value_in.device());
   Tensor value = value_in;
   if (reinterpret_cast<uintptr_t>(value.data_ptr()) % 16)  // the kernel reads 16-byte rows
@@ -139,6 +145,7 @@ std::tuple<Tensor, Tensor> quantize_mxfp8_dynamic(const Tensor& value_in, bool s
 }
 
 std::tuple<Tensor, Tensor> quantize_int8_rows(const Tensor& value, bool reciprocal) {
+  check_dims(value, 2, "quantize_int8_rows");
   const c10::DeviceGuard guard(value.device());
   const int64_t rows = value.size(0), k = value.size(1);
   Tensor q = empty({rows, k}, value, at::kChar), scale = empty({rows}, value, at::kFloat);
@@ -149,6 +156,7 @@ std::tuple<Tensor, Tensor> quantize_int8_rows(const Tensor& value, bool reciproc
 }
 
 Tensor calibrate_block32(const Tensor& matrix) {
+  check_dims(matrix, 2, "calibrate_block32");
   const c10::DeviceGuard guard(matrix.device());
   const int64_t rows = matrix.size(0), channels = matrix.size(1), groups = (channels + BLOCK - 1) / BLOCK;
   Tensor workspace = empty({groups}, matrix, at::kInt), exponent = empty({groups}, matrix, at::kChar);
@@ -192,6 +200,8 @@ struct Geometry {
 Tensor int8_conv2d(const Tensor& x, const Tensor& weight, const Tensor& a_scale, const Tensor& w_scale,
                    const OptTensor& bias, FIM_GEO_PARAMS, bool relu, bool gelu, const OptTensor& residual,
                    const OptTensor& out_scale) {
+  check_dims(x, 4, "int8_conv2d");
+  TORCH_CHECK_INDEX(!residual || residual->dim() <= 4, "int8_conv2d: residual of shape ", residual->sizes());
   const c10::DeviceGuard guard(x.device());
   const Geometry g = FIM_GEO;
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), cin = x.size(3), cout = weight.size(0);
@@ -209,6 +219,7 @@ Tensor int8_conv2d(const Tensor& x, const Tensor& weight, const Tensor& a_scale,
 std::tuple<Tensor, Tensor> int8_conv2d_maxpool(const Tensor& x, const Tensor& weight, const Tensor& a_scale,
                                                const Tensor& w_scale, const OptTensor& bias, FIM_GEO_PARAMS, bool relu,
                                                const Tensor& out_scale) {
+  check_dims(x, 4, "int8_conv2d_maxpool");
   const c10::DeviceGuard guard(x.device());
   const Geometry g = FIM_GEO;
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), cin = x.size(3), cout = weight.size(0);
@@ -226,6 +237,8 @@ std::tuple<Tensor, Tensor> int8_conv2d_maxpool(const Tensor& x, const Tensor& we
 Tensor mxfp8_conv2d(const Tensor& x, const Tensor& channel_exponent, const Tensor& weight, const Tensor& weight_exponent,
                     const OptTensor& bias, FIM_GEO_PARAMS, bool relu, bool gelu, const OptTensor& residual,
                     const OptTensor& out_exponent) {
+  check_dims(x, 4, "mxfp8_conv2d");
+  TORCH_CHECK_INDEX(!residual || residual->dim() <= 4, "mxfp8_conv2d: residual of shape ", residual->sizes());
   const c10::DeviceGuard guard(x.device());
   const Geometry g = FIM_GEO;
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), cin = x.size(3), cout = weight.size(0);
@@ -242,6 +255,7 @@ Tensor mxfp8_conv2d(const Tensor& x, const Tensor& channel_exponent, const Tenso
 
 Tensor int8_linear(const Tensor& a, const Tensor& weight, const Tensor& a_scale, const Tensor& w_scale,
                    const OptTensor& bias, bool relu, bool gelu, const OptTensor& residual) {
+  check_dims(a, 2, "int8_linear");
   const c10::DeviceGuard guard(a.device());
   const int64_t m = a.size(0), k = a.size(1), n = weight.size(0);
   const bool per_row = a_scale.numel() != 1;
@@ -257,6 +271,7 @@ Tensor int8_linear(const Tensor& a, const Tensor& weight, const Tensor& a_scale,
 
 void int8_linear_quantize_(const Tensor& a, const Tensor& weight, const Tensor& a_scale, const Tensor& w_scale,
                            const OptTensor& bias, const Tensor& out_scale, const Tensor& out) {
+  check_dims(a, 2, "int8_linear_quantize_");
   const c10::DeviceGuard guard(a.device());
   const int64_t m = a.size(0), k = a.size(1), n = weight.size(0);
   const bool per_row = a_scale.numel() != 1;
@@ -270,6 +285,7 @@ void int8_linear_quantize_(const Tensor& a, const Tensor& weight, const Tensor& 
 
 Tensor mxfp8_scaled_mm(const Tensor& a, const Tensor& a_scale_swizzled, const Tensor& weight,
                        const Tensor& weight_exponent, const OptTensor& bias, bool weight_scale_e8m0) {
+  check_dims(a, 2, "mxfp8_scaled_mm");
   const c10::DeviceGuard guard(a.device());
   const int64_t m = a.size(0), k = a.size(1), n = weight.size(0);
   Tensor out = empty({m, n}, a, at::kBFloat16);
@@ -281,6 +297,7 @@ Tensor mxfp8_scaled_mm(const Tensor& a, const Tensor& a_scale_swizzled, const Te
 }
 
 Tensor im2col_gather(const Tensor& x, FIM_GEO_PARAMS) {
+  check_dims(x, 4, "im2col_gather");
   const c10::DeviceGuard guard(x.device());
   const Geometry g = FIM_GEO;
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), c = x.size(3);
@@ -294,6 +311,7 @@ Tensor im2col_gather(const Tensor& x, FIM_GEO_PARAMS) {
 Tensor refiner_mlp(int64_t kind, int64_t semantics, const Tensor& x, const Tensor& x_scale, const Tensor& w1,
                    const Tensor& w1_scale, const OptTensor& b1, const Tensor& h_scale, const Tensor& w2,
                    const Tensor& w2_scale, const OptTensor& b2, const OptTensor& residual) {
+  check_dims(x, 2, "refiner_mlp");
   const c10::DeviceGuard guard(x.device());
   const int64_t rows = x.size(0), c = x.size(1), h = w1.size(0);
   Tensor out = empty({rows, w2.size(0)}, x, at::kBFloat16);
@@ -309,6 +327,7 @@ constexpr int DW_MX_DYNAMIC = 0, DW_INT8 = 1, DW_BF16 = 2, DW_MX_STATIC = 3;
 
 Tensor depthwise5x5(const Tensor& x, const Tensor& weight, const Tensor& bias, int64_t act, int64_t mode,
                     const OptTensor& scale, const OptTensor& exponent) {
+  check_dims(x, 4, "depthwise5x5");
   const c10::DeviceGuard guard(x.device());
   TORCH_CHECK(mode == DW_INT8 || mode == DW_BF16 || mode == DW_MX_STATIC, "depthwise5x5: no output mode ", mode);
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), c = x.size(3);
@@ -321,6 +340,7 @@ Tensor depthwise5x5(const Tensor& x, const Tensor& weight, const Tensor& bias, i
 }
 
 std::tuple<Tensor, Tensor> depthwise5x5_mx_dynamic(const Tensor& x, const Tensor& weight, const Tensor& bias) {
+  check_dims(x, 4, "depthwise5x5_mx_dynamic");
   const c10::DeviceGuard guard(x.device());
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), c = x.size(3), rows = b * h * w;
   Tensor out = empty({rows, c}, x, at::kByte), swz = swizzled_scales(rows, c / BLOCK, x);
@@ -333,6 +353,7 @@ std::tuple<Tensor, Tensor> depthwise5x5_mx_dynamic(const Tensor& x, const Tensor
 
 Tensor depthwise5x5_relu_pointwise_mxfp8(const Tensor& x, const Tensor& dw_weight, const Tensor& dw_bias,
                                          const Tensor& pw_weight, const Tensor& pw_e8m0, const OptTensor& pw_bias) {
+  check_dims(x, 4, "depthwise5x5_relu_pointwise_mxfp8");
   const c10::DeviceGuard guard(x.device());
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), c = x.size(3), n = pw_weight.size(0);
   Tensor out = empty({b, h, w, n}, x, at::kBFloat16);
@@ -347,6 +368,7 @@ Tensor depthwise5x5_relu_pointwise_mxfp8(const Tensor& x, const Tensor& dw_weigh
 Tensor depthwise5x5_relu_pointwise_int8(const Tensor& x, const Tensor& dw_weight, const Tensor& dw_bias,
                                         const Tensor& scale, const Tensor& pw_weight, const Tensor& pw_wscale,
                                         const OptTensor& pw_bias) {
+  check_dims(x, 4, "depthwise5x5_relu_pointwise_int8");
   const c10::DeviceGuard guard(x.device());
   const int64_t b = x.size(0), h = x.size(1), w = x.size(2), c = x.size(3), n = pw_weight.size(0);
   Tensor out = empty({b, h, w, n}, x, at::kBFloat16);
@@ -360,6 +382,7 @@ Tensor depthwise5x5_relu_pointwise_int8(const Tensor& x, const Tensor& dw_weight
 }
 
 Tensor conv3x3_small_cin_quantize_int8(const Tensor& x, const Tensor& packed, const Tensor& bias, const Tensor& scale) {
+  check_dims(x, 4, "conv2d_small_cin_quantize_int8");
   const c10::DeviceGuard guard(x.device());
   const int64_t b = x.size(0), cin = x.size(1), h = x.size(2), w = x.size(3), cout = packed.size(0);
   Tensor out = empty({b, h, w, cout}, x, at::kChar);
@@ -371,6 +394,7 @@ Tensor conv3x3_small_cin_quantize_int8(const Tensor& x, const Tensor& packed, co
 }
 
 Tensor bias_relu_quantize_int8(const Tensor& raw, const Tensor& bias, const Tensor& scale) {
+  check_dims(raw, 4, "bias_relu_quantize_int8");
   const c10::DeviceGuard guard(raw.device());
   const int64_t b = raw.size(0), c = raw.size(1), h = raw.size(2), w = raw.size(3);
   Tensor out = empty({b, h, w, c}, raw, at::kChar);
@@ -381,6 +405,7 @@ Tensor bias_relu_quantize_int8(const Tensor& raw, const Tensor& bias, const Tens
 }
 
 Tensor pointwise_bf16(const Tensor& x, const Tensor& weight, const OptTensor& bias) {
+  check_dims(x, 2, "pointwise_bf16");
   const c10::DeviceGuard guard(x.device());
   const int64_t m = x.size(0), k = x.size(1), n = weight.size(0);
   Tensor out = empty({m, n}, x, at::kBFloat16);

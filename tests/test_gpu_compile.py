@@ -85,3 +85,66 @@ def test_backward_through_an_op_raises():
     y = torch.ops.flashim_amd.depthwise5x5(x, w, b, 1, 2, None, None)
     with pytest.raises(RuntimeError, match="not implemented"):
         y.float().sum().backward()
+
+
+def _zeros(*shape, dtype=torch.int8):
+    return torch.zeros(shape, device=DEV, dtype=dtype)
+
+
+GEO3 = (3, 3, 1, 1, 1, 1, 1, 1)
+_F32, _BF16, _U8 = torch.float32, torch.bfloat16, torch.uint8
+# op, its arguments with an input of the shape the op takes, the index of that input
+RANKS = {
+    "quantize_mxfp8_dynamic": lambda: [_zeros(32, 32, dtype=_F32), True],
+    "quantize_int8_rows": lambda: [_zeros(32, 32, dtype=_F32), True],
+    "calibrate_block32": lambda: [_zeros(32, 32, dtype=_F32)],
+    "int8_conv2d": lambda: [_zeros(2, 8, 8, 32), _zeros(32, 288), _zeros(1, dtype=_F32), _zeros(32, dtype=_F32), None,
+                            *GEO3, False, False, None, None],
+    "int8_conv2d_maxpool": lambda: [_zeros(2, 8, 8, 32), _zeros(32, 288), _zeros(1, dtype=_F32),
+                                    _zeros(32, dtype=_F32), None, *GEO3, False, torch.ones(1, device=DEV)],
+    "mxfp8_conv2d": lambda: [_zeros(2, 8, 8, 32, dtype=_U8), _zeros(1), _zeros(32, 288, dtype=_U8), _zeros(32, 9), None,
+                             *GEO3, False, False, None, None],
+    "int8_linear": lambda: [_zeros(32, 32), _zeros(32, 32), _zeros(1, dtype=_F32), _zeros(32, dtype=_F32), None, False,
+                            False, None],
+    "int8_linear_quantize_": lambda: [_zeros(32, 32), _zeros(32, 32), _zeros(1, dtype=_F32), _zeros(32, dtype=_F32),
+                                      None, torch.ones(1, device=DEV), _zeros(32, 32)],
+    "mxfp8_scaled_mm": lambda: [_zeros(32, 32, dtype=_U8), _zeros(512, dtype=_U8), _zeros(32, 32, dtype=_U8),
+                                _zeros(32, 1), None],
+    "im2col_gather": lambda: [_zeros(2, 8, 8, 32, dtype=_U8), *GEO3],
+    "refiner_mlp": lambda: [0, 0, _zeros(32, 64), _zeros(1, dtype=_F32), _zeros(256, 64), _zeros(256, dtype=_F32), None,
+                            torch.ones(1, device=DEV), _zeros(64, 256), _zeros(64, dtype=_F32), None, None],
+    "depthwise5x5": lambda: [_zeros(2, 8, 8, 32, dtype=_BF16), _zeros(25, 32, dtype=_BF16), _zeros(32, dtype=_F32), 0, 2,
+                             None, None],
+    "depthwise5x5_mx_dynamic": lambda: [_zeros(2, 8, 8, 32, dtype=_BF16), _zeros(25, 32, dtype=_BF16),
+                                        _zeros(32, dtype=_F32)],
+    "conv3x3_small_cin_quantize_int8": lambda: [_zeros(2, 3, 8, 8, dtype=_BF16), _zeros(16, 32, dtype=_BF16),
+                                                _zeros(16, dtype=_F32), torch.ones(1, device=DEV)],
+    "bias_relu_quantize_int8": lambda: [_zeros(2, 16, 8, 8, dtype=_BF16), _zeros(16, dtype=_F32),
+                                        torch.ones(1, device=DEV)],
+    "pointwise_bf16": lambda: [_zeros(32, 32, dtype=_BF16), _zeros(32, 32, dtype=_BF16), None],
+}
+
+
+@pytest.mark.parametrize("name", RANKS)
+def test_ops_refuse_inputs_of_another_rank(name):
+    """The ops read leading sizes only, so an input of one dimension more would be taken for its first dimensions (a
+    [2, 32, 32] as [2, 32]): they raise ValueError before anything is allocated or launched."""
+    op = getattr(torch.ops.flashim_amd, name)
+    args = RANKS[name]()
+    op(*args)
+    at = 2 if name == "refiner_mlp" else 0
+    for wrong in (args[at].unsqueeze(0), args[at][0]):
+        with pytest.raises(ValueError, match="dimensions"):
+            op(*args[:at], wrong, *args[at + 1:])
+
+
+def test_int8_rows_of_a_3d_tensor_are_refused():
+    for fn in (quant.quantize_int8_rows, quant.weight_scales_and_values, quant.quantize_dynamic_2d):
+        with pytest.raises(ValueError):
+            fn(torch.randn(2, 32, 32, device=DEV))
+
+
+def test_conv_residual_of_five_dimensions_is_refused():
+    args = RANKS["int8_conv2d"]()
+    with pytest.raises(IndexError):
+        torch.ops.flashim_amd.int8_conv2d(*args[:-2], _zeros(1, 2, 8, 8, 32, dtype=_BF16), None)
