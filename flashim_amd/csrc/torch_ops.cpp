@@ -13,6 +13,7 @@
 #include <optional>
 #include <string>
 #include <tuple>
+#include <vector>
 
 #include "../../include/flashim_amd.h"
 
@@ -70,17 +71,22 @@ struct View4 {
       n[pad + i] = t.size(i);
       s[pad + i] = t.stride(i);
     }
-    for (int64_t i = pad - 1; i >= 0; --i) s[i] = n[i + 1] * s[i + 1];  // as unsqueeze does
+    for (int64_t i = pad - 1; i >= 0; --i) s[i] = i == 3 ? 1 : n[i + 1] * s[i + 1];  // as unsqueeze does (i = 3: no dimensions)
   }
 };
 
 #define FIM_VIEW4(v) v.n[0], v.n[1], v.n[2], v.n[3], v.s[0], v.s[1], v.s[2], v.s[3]
 
+std::vector<int64_t> padded_sizes(const Tensor& value, int64_t padded) {
+  auto sizes = value.sizes().vec();
+  if (!sizes.empty()) sizes.pop_back();
+  sizes.push_back(padded);
+  return sizes;
+}
+
 Tensor quantize_mxfp8(const Tensor& value, const Tensor& exponent, int64_t padded) {
   const c10::DeviceGuard guard(value.device());
-  auto sizes = value.sizes().vec();
-  sizes.back() = padded;
-  Tensor out = empty(sizes, value, at::kByte);
+  Tensor out = empty(padded_sizes(value, padded), value, at::kByte);
   const View4 v(value);
   check(fim_quantize_mxfp8(v.t.data_ptr(), dtype_code(value), FIM_VIEW4(v), ptr<const int8_t>(exponent),
                            ptr<uint8_t>(out), padded, stream_of(value)),
@@ -91,9 +97,7 @@ Tensor quantize_mxfp8(const Tensor& value, const Tensor& exponent, int64_t padde
 Tensor gelu_quantize_mxfp8(const Tensor& value, const Tensor& exponent, int64_t padded, const OptTensor& input_bias,
                            bool tanh) {
   const c10::DeviceGuard guard(value.device());
-  auto sizes = value.sizes().vec();
-  sizes.back() = padded;
-  Tensor out = empty(sizes, value, at::kByte);
+  Tensor out = empty(padded_sizes(value, padded), value, at::kByte);
   const View4 v(value);
   check(fim_gelu_quantize_mxfp8(v.t.data_ptr(), dtype_code(value), FIM_VIEW4(v), tanh, ptr<const float>(input_bias),
                                 ptr<const int8_t>(exponent), ptr<uint8_t>(out), padded, stream_of(value)),

@@ -139,3 +139,16 @@ def test_calibrate_block32(shape):
     x = torch.randn(shape) * 10 * torch.rand(shape[-1])
     got = quant.calibrate_block32_exponent(x.to(DEV))
     assert torch.equal(got.cpu(), ref.calibrate_block32_exponent(x))
+
+
+def test_zero_dimensional_values():
+    """A 0-d tensor is one channel: the operators take it as [1, 1, 1, 1]."""
+    value, scale = torch.tensor(1.3, device=DEV), torch.tensor(0.02, device="cuda")
+    got = quant.quantize_int8_static(value, scale).values
+    assert got.shape == () and torch.equal(got.cpu(), ref.quantize_int8_static(value.cpu(), scale.cpu()))
+    assert torch.equal(quant.gelu_quantize_int8_static(value, scale).values,
+                       quant.gelu_quantize_int8_static(value.reshape(1), scale).values[0])
+    exponent = torch.zeros(1, device=DEV, dtype=torch.int8)
+    for op, extra in ((torch.ops.flashim_amd.quantize_mxfp8, ()), (torch.ops.flashim_amd.gelu_quantize_mxfp8, (None,))):
+        codes = op(value, exponent, 32, *extra)
+        assert codes.shape == (32,) and torch.equal(codes, op(value.reshape(1, 1), exponent, 32, *extra)[0])
