@@ -7,6 +7,8 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/library.h>
 
 #include <array>
@@ -471,9 +473,41 @@ TORCH_LIBRARY_IMPL(flashim_amd, CUDA, m) {
 #undef X
 }
 
-// no derivative formulas: a backward pass through an op raises
+namespace {
+
+// No derivative formulas. Reverse mode: the outputs of inputs that require a gradient carry a node that raises. Forward
+// mode alone: the tangents of dual inputs stop here and the outputs have none (torch's own fallback for operators without
+// formulas refuses every dual input).
+void no_derivative(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit::Stack* stack) {
+  const std::string& name = op.schema().name();
+  torch::autograd::variable_list inputs;  // that require a gradient
+  if (at::GradMode::is_enabled()) {
+    bool dual = false;
+    for (const c10::IValue& arg : torch::jit::last(*stack, op.schema().arguments().size()))
+      if (arg.isTensor()) {
+        const Tensor& t = arg.toTensor();
+        if (t.requires_grad()) inputs.push_back(t);
+        dual = dual || torch::autograd::isFwGradDefined(t);
+      }
+    TORCH_CHECK_NOT_IMPLEMENTED(inputs.empty() || !dual, name,
+                                ": no forward-mode derivative, and an input requires a gradient");
+  }
+  {
+    at::AutoDispatchBelowAutograd guard;
+    op.redispatchBoxed(keys & c10::after_autograd_keyset, stack);
+  }
+  if (inputs.empty()) return;
+  std::shared_ptr<torch::autograd::Node> node(new torch::autograd::NotImplemented(name), torch::autograd::deleteNode);
+  node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+  for (const c10::IValue& out : torch::jit::last(*stack, op.schema().returns().size()))
+    if (out.isTensor() && torch::autograd::isDifferentiableType(out.toTensor().scalar_type()))
+      torch::autograd::set_history(out.toTensor(), node);
+}
+
+}  // namespace
+
 TORCH_LIBRARY_IMPL(flashim_amd, Autograd, m) {
-#define X(name, schema) m.impl(#name, torch::autograd::autogradNotImplementedFallback());
+#define X(name, schema) m.impl(#name, torch::CppFunction::makeFromBoxedFunction<&no_derivative>());
   FIM_OPS(X)
 #undef X
 }

@@ -5,6 +5,7 @@ dtypes the oracle's real outputs have for the same inputs. This is what ``torch.
 
 import pytest
 import torch
+from torch.autograd import forward_ad
 from torch._subclasses.fake_tensor import FakeTensorMode
 
 from flashim_amd import quant
@@ -141,3 +142,27 @@ def test_ops_without_a_gpu_kernel_or_derivative_refuse():
         w, b = torch.empty(25, 32, device="cuda", dtype=torch.bfloat16), torch.empty(32, device="cuda")
         y = torch.ops.flashim_amd.depthwise5x5(x, w, b, 1, 2, None, None)
         assert y.requires_grad and "NotImplemented" in type(y.grad_fn).__name__ + y.grad_fn.name()
+
+
+def test_forward_mode_inputs_pass_without_tangents():
+    """A dual input goes in by its value and the outputs carry no tangent; with an input that requires a gradient as well
+    the op raises."""
+    x = torch.empty(1, 8, 8, 32, device="meta", dtype=torch.bfloat16)
+    w, b = torch.empty(25, 32, device="meta", dtype=torch.bfloat16), torch.empty(32, device="meta")
+
+    def depthwise(x, w):
+        return torch.ops.flashim_amd.depthwise5x5(x, w, b, 1, 2, None, None)
+
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(x, torch.empty_like(x))
+        assert forward_ad.unpack_dual(depthwise(dual, w)).tangent is None
+        assert torch.ops.flashim_amd.quantize_int8(dual, torch.empty(1, device="meta"), None).dtype == torch.int8
+        codes, scales = torch.ops.flashim_amd.depthwise5x5_mx_dynamic(dual, w, b)
+        assert codes.dtype == scales.dtype == torch.uint8
+        w_grad = w.clone().requires_grad_()
+        with pytest.raises(NotImplementedError):
+            depthwise(dual, w_grad)
+        with torch.no_grad():
+            assert not depthwise(dual, w_grad).requires_grad
+    y, tangent = torch.func.jvp(lambda v: depthwise(v, w), (x,), (torch.empty_like(x),))
+    assert y.shape == tangent.shape == (64, 32)
