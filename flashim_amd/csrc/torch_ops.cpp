@@ -6,7 +6,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
-#include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
+#include <torch/csrc/autograd/VariableTypeUtils.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/library.h>
@@ -73,7 +73,7 @@ struct View4 {
       n[pad + i] = t.size(i);
       s[pad + i] = t.stride(i);
     }
-    for (int64_t i = pad - 1; i >= 0; --i) s[i] = i == 3 ? 1 : n[i + 1] * s[i + 1];  // as unsqueeze does (i = 3: no dimensions)
+    for (int64_t i = pad - 1; i >= 0; --i) s[i] = i == 3 ? 1 : n[i + 1] * s[i + 1];  // as unsqueeze does
   }
 };
 
@@ -504,6 +504,17 @@ void no_derivative(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torc
       torch::autograd::set_history(out.toTensor(), node);
 }
 
+// The version counter of the last argument, the tensor that is written, by which autograd finds a saved tensor that was
+// overwritten since (torch's own fallback counts for returned tensors only).
+void count_write_to_last(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit::Stack* stack) {
+  const Tensor out = stack->back().toTensor();
+  {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    op.redispatchBoxed(keys & c10::after_ADInplaceOrView_keyset, stack);
+  }
+  if (!out.is_inference()) torch::autograd::increment_version(out);
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(flashim_amd, Autograd, m) {
@@ -513,5 +524,5 @@ TORCH_LIBRARY_IMPL(flashim_amd, Autograd, m) {
 }
 
 TORCH_LIBRARY_IMPL(flashim_amd, ADInplaceOrView, m) {
-  m.impl("int8_linear_quantize_", torch::autograd::autogradNotImplementedInplaceOrViewFallback());
+  m.impl("int8_linear_quantize_", torch::CppFunction::makeFromBoxedFunction<&count_write_to_last>());
 }

@@ -166,3 +166,27 @@ def test_forward_mode_inputs_pass_without_tangents():
             assert not depthwise(dual, w_grad).requires_grad
     y, tangent = torch.func.jvp(lambda v: depthwise(v, w), (x,), (torch.empty_like(x),))
     assert y.shape == tangent.shape == (64, 32)
+
+
+def _linear_quantize_into(out):
+    torch.ops.flashim_amd.int8_linear_quantize_(
+        torch.empty(16, 32, device="meta", dtype=torch.int8), torch.empty(32, 32, device="meta", dtype=torch.int8),
+        torch.empty(1, device="meta"), torch.empty(32, device="meta"), None, torch.empty(1, device="meta"), out)
+
+
+def test_in_place_op_bumps_the_version_of_what_it_writes():
+    """Autograd finds a saved tensor that was overwritten by its version counter (inference tensors have none)."""
+    base = torch.empty(16, 64, device="meta", dtype=torch.int8)
+    for out in (torch.empty(16, 32, device="meta", dtype=torch.int8), base[:, :32]):
+        _linear_quantize_into(out)
+        assert out._version == 1
+    assert base._version == 1
+    x = torch.empty(16, 64, device="meta", requires_grad=True)
+    y = x * base  # saves base
+    _linear_quantize_into(base[:, :32])
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+    with torch.inference_mode():
+        out = torch.empty(16, 32, device="meta", dtype=torch.int8)
+        _linear_quantize_into(out)
+    _linear_quantize_into(out)
