@@ -47,13 +47,17 @@ def _run(cmd: list[str]) -> None:
 
 
 def build_torch_ops() -> Path:
-    """Compile ``csrc/torch_ops.cpp`` against the installed torch and link it to ``libflashim_amd.so`` beside it."""
+    """Compile ``csrc/torch_ops.cpp`` against the installed torch and link it to ``libflashim_amd.so`` beside it (Python's
+    own symbols come from the interpreter that loads it)."""
+    import sysconfig
+
     import torch
     from torch.utils import cpp_extension
 
     temporary = TORCH_LIBRARY.with_suffix(f".{os.getpid()}.tmp")
     torch_lib = Path(torch.__file__).parent / "lib"
-    includes = [flag for path in cpp_extension.include_paths("cuda") for flag in ("-isystem", path)]
+    includes = [flag for path in (*cpp_extension.include_paths("cuda"), sysconfig.get_path("include"))
+                for flag in ("-isystem", path)]
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, str(CSRC / "torch_ops.cpp"),
           "-o", str(temporary), f"-L{PACKAGE}", "-lflashim_amd", f"-L{torch_lib}", "-lc10", "-ltorch_cpu", "-lc10_hip",

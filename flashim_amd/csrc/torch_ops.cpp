@@ -6,6 +6,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
 #include <torch/csrc/autograd/VariableTypeUtils.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -45,11 +46,18 @@ int dtype_code(const Tensor& t) {
 int bias_code(const Tensor& t) { return t.scalar_type() == at::kBFloat16 ? 1 : 0; }
 int bias_code(const OptTensor& t) { return t && t->scalar_type() == at::kBFloat16 ? 1 : 0; }
 
-// library.py turns the text of status 99 into its own exception type
+// Status 99 as the package's own exception, raised here so that compiled graphs, which call the operators themselves, see
+// its type too.
+[[noreturn]] void raise_unsupported(const std::string& message) {
+  pybind11::gil_scoped_acquire gil;
+  PyErr_SetString(pybind11::module_::import("flashim_amd._lib").attr("UnsupportedShape").ptr(), message.c_str());
+  throw pybind11::error_already_set();
+}
+
 template <typename... What>
 void check(int code, const What&... what) {
   if (code == FIM_OK) return;
-  TORCH_CHECK(code != FIM_ERR_UNSUPPORTED, what..., ": no HIP kernel for this shape/layout (code 99)");
+  if (code == FIM_ERR_UNSUPPORTED) raise_unsupported(c10::str(what..., ": no HIP kernel for this shape/layout (code 99)"));
   TORCH_CHECK(false, what..., " launch failed (code ", code, ")");
 }
 

@@ -3,8 +3,8 @@ instead of breaking its graph at every call into the library (the pattern of Fla
 ``flashim/backends/cuda/conv.py:55-76, 148-161``).
 
 The ops are defined and implemented in C++ (``csrc/torch_ops.cpp``: outputs from torch's caching allocator, one C call on
-the current stream, an exception on a nonzero status), registered when ``libflashim_amd_torch.so`` is loaded; their fakes,
-which return empty outputs of the same shape, dtype and device, are here. Arguments arrive normalized by the impls in
+the current stream, an exception on a nonzero status, :class:`flashim_amd._lib.UnsupportedShape` for 99), registered when
+``libflashim_amd_torch.so`` is loaded; their fakes, which return empty outputs of the same shape, dtype and device, are here. Arguments arrive normalized by the impls in
 :mod:`flashim_amd.backends.hip` (dtypes, contiguity, devices): the bodies only read pointers, sizes and strides.
 """
 
@@ -15,7 +15,6 @@ from collections.abc import Callable
 
 import torch
 
-from flashim_amd import _lib
 from flashim_amd._build import TORCH_LIBRARY
 
 NS = "flashim_amd"
@@ -45,19 +44,12 @@ def _load() -> None:
 
 
 def _op(name: str) -> Callable:
-    """The op as a function that loads the library on first use; status 99 raises ``UnsupportedShape``."""
+    """The op as a function that loads the library on first use."""
 
     def call(*args, **kwargs):
         if name not in _OVERLOADS:
             _load()
-        if torch.compiler.is_compiling():
-            return _OVERLOADS[name](*args, **kwargs)
-        try:
-            return _OVERLOADS[name](*args, **kwargs)
-        except RuntimeError as error:
-            if "no HIP kernel for this shape/layout (code 99)" in str(error):
-                raise _lib.UnsupportedShape(str(error)) from None
-            raise
+        return _OVERLOADS[name](*args, **kwargs)
 
     call.__name__ = name
     return call

@@ -5,7 +5,7 @@ through this package's dispatcher, as FlashIM's region compile would through its
 import pytest
 import torch
 
-from flashim_amd import ops, quant
+from flashim_amd import _lib, ops, quant
 from oracle import reference as ref
 
 pytestmark = pytest.mark.gpu
@@ -148,3 +148,13 @@ def test_conv_residual_of_five_dimensions_is_refused():
     args = RANKS["int8_conv2d"]()
     with pytest.raises(IndexError):
         torch.ops.flashim_amd.int8_conv2d(*args[:-2], _zeros(1, 2, 8, 8, 32, dtype=_BF16), None)
+
+
+def test_unsupported_shapes_raise_their_own_type_compiled_too():
+    """The BF16 pointwise kernel takes up to 128 output channels: status 99 from the library."""
+    x, weight = _zeros(32, 32, dtype=_BF16), _zeros(144, 32, dtype=_BF16)
+    op = torch.ops.flashim_amd.pointwise_bf16
+    torch._dynamo.reset()
+    for fn in (op, torch.compile(lambda x: op(x, weight, None), fullgraph=True)):
+        with pytest.raises(_lib.UnsupportedShape, match="no HIP kernel"):
+            fn(x, weight, None) if fn is op else fn(x)
