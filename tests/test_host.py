@@ -12,7 +12,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from flashim_amd import _lib, blocks, dispatch, ops, quant
+from flashim_amd import _build, _lib, blocks, dispatch, ops, quant
 from flashim_amd.platforms import Feature, Platform, rocm_features
 from oracle import reference as ref
 
@@ -187,6 +187,15 @@ def test_host_int8_quotient_rounds_as_the_division(scale):
     x = torch.cat([x[~x.isnan()], near[near.isfinite()]])
     got = _call(h.fim_host_int8_quotient, x.numpy(), np.int8, ctypes.c_float(scale))
     assert np.array_equal(got, (x / s).round().clamp(-127, 127).to(torch.int8).numpy())
+
+
+# -- what an installed package holds and how it loads ----------------------------------------------------------------
+
+
+def test_package_data_lists_the_libraries_a_call_needs():
+    tomli = pytest.importorskip("tomli")
+    listed = tomli.loads((ROOT / "pyproject.toml").read_text())["tool"]["setuptools"]["package-data"]["flashim_amd"]
+    assert {_build.LIBRARY.name, _build.TORCH_LIBRARY.name} <= set(listed)
 
 
 # -- the dispatcher ----------------------------------------------------------------------------------------------
