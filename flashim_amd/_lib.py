@@ -131,8 +131,12 @@ def probe_call(name: str, *args, what: str | None = None) -> None:
 
 
 def available() -> bool:
+    """Whether a call can reach the kernels: the HIP library and the torch operators on it are built and load."""
+    from flashim_amd import library
+
     try:
         load()
+        library.load()
         return True
     except (RuntimeError, OSError):
         return False

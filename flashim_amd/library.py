@@ -27,7 +27,7 @@ _OVERLOADS: dict[str, Callable] = {}
 _lock = threading.Lock()
 
 
-def _load() -> None:
+def load() -> None:
     """Load the op library and register the fakes, once. Raises if it has not been built."""
     with _lock:
         if _OVERLOADS:
@@ -48,7 +48,7 @@ def _op(name: str) -> Callable:
 
     def call(*args, **kwargs):
         if name not in _OVERLOADS:
-            _load()
+            load()
         return _OVERLOADS[name](*args, **kwargs)
 
     call.__name__ = name
@@ -230,4 +230,4 @@ def pointwise_bf16(x, weight, bias):
 
 
 if TORCH_LIBRARY.is_file():  # ``torch.ops.flashim_amd`` is there on import; a library built later is loaded on first use
-    _load()
+    load()

@@ -12,7 +12,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from flashim_amd import _build, _lib, blocks, dispatch, ops, quant
+from flashim_amd import _build, _lib, blocks, dispatch, library, ops, quant
 from flashim_amd.platforms import Feature, Platform, rocm_features
 from oracle import reference as ref
 
@@ -196,6 +196,17 @@ def test_package_data_lists_the_libraries_a_call_needs():
     tomli = pytest.importorskip("tomli")
     listed = tomli.loads((ROOT / "pyproject.toml").read_text())["tool"]["setuptools"]["package-data"]["flashim_amd"]
     assert {_build.LIBRARY.name, _build.TORCH_LIBRARY.name} <= set(listed)
+
+
+def test_available_needs_the_torch_operators_too(monkeypatch, tmp_path):
+    """FlashIM's references stay the fallback where a call into the HIP impls could not load what it needs."""
+    assert _lib.available()
+    damaged = tmp_path / _build.TORCH_LIBRARY.name
+    damaged.write_bytes(b"not a library")
+    for path in (tmp_path / "missing.so", damaged):
+        monkeypatch.setattr(library, "TORCH_LIBRARY", path)
+        monkeypatch.setattr(library, "_OVERLOADS", {})
+        assert not _lib.available()
 
 
 # -- the dispatcher ----------------------------------------------------------------------------------------------
