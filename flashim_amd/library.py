@@ -10,12 +10,15 @@ the current stream, an exception on a nonzero status, :class:`flashim_amd._lib.U
 
 from __future__ import annotations
 
+import logging
 import threading
 from collections.abc import Callable
 
 import torch
 
 from flashim_amd._build import TORCH_LIBRARY
+
+logger = logging.getLogger(__name__)
 
 NS = "flashim_amd"
 BLOCK = 32
@@ -229,5 +232,10 @@ def pointwise_bf16(x, weight, bias):
     return x.new_empty((x.shape[0], weight.shape[0]), dtype=torch.bfloat16)
 
 
-if TORCH_LIBRARY.is_file():  # ``torch.ops.flashim_amd`` is there on import; a library built later is loaded on first use
-    load()
+# ``torch.ops.flashim_amd`` is there on import. A library that is built later is loaded on first use, and so is one that
+# does not load now (built against another torch, a missing HIP runtime): the first op raises the loader's error.
+if TORCH_LIBRARY.is_file():
+    try:
+        load()
+    except OSError as error:
+        logger.warning("%s does not load: %s", TORCH_LIBRARY, error)

@@ -4,7 +4,11 @@ the host build of the kernels' scalar numerics matches torch exhaustively, the d
 no-fallback rule, and the host-side layout / packing helpers."""
 
 import ctypes
+import os
 import re
+import shutil
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -207,6 +211,26 @@ def test_available_needs_the_torch_operators_too(monkeypatch, tmp_path):
         monkeypatch.setattr(library, "TORCH_LIBRARY", path)
         monkeypatch.setattr(library, "_OVERLOADS", {})
         assert not _lib.available()
+
+
+def test_import_survives_an_operator_library_that_does_not_load(tmp_path):
+    """A library built against another torch fails at first use, with the loader's own error, not at import."""
+    package = tmp_path / "flashim_amd"
+    shutil.copytree(ROOT / "flashim_amd", package, ignore=shutil.ignore_patterns("*.so", "_build", "csrc", "__pycache__"))
+    (package / _build.TORCH_LIBRARY.name).write_bytes(b"not a library")
+    script = """
+import torch
+import flashim_amd.ops, flashim_amd.plugin
+from flashim_amd import _lib, library
+assert not _lib.available()
+try:
+    library.quantize_int8(torch.zeros(4, 32), torch.ones(1), None)
+except OSError as error:
+    print("first use:", error)
+"""
+    run = subprocess.run([sys.executable, "-c", script], cwd=tmp_path, capture_output=True, text=True, timeout=300,
+                         env={**os.environ, "PYTHONPATH": str(tmp_path)})
+    assert run.returncode == 0 and "first use:" in run.stdout, run.stderr
 
 
 # -- the dispatcher ----------------------------------------------------------------------------------------------
