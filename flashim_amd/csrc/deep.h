@@ -40,9 +40,8 @@ __global__ __launch_bounds__(256, TWO ? 2 : 1) void conv_deep_kernel(const DeepA
   constexpr int WM = 4 / WN, BR = DEEP_BR;
   constexpr int BM = WM * MBW * BR, BN = WN * 64;
   // a stage: the weight rows, then the activation rows, in 8-row chunks (one wave-wide 16-byte-per-lane load each);
-  // wavefront w loads chunks w, w + 4, ... of each (where the activation chunks, an even number, end in half a round of
-  // four, wavefronts 2 and 3 load wavefront 0's and 1's again)
-  constexpr int ACH = BM / 8, NW = BN / 32, NA = (ACH + 3) / 4, CHUNKS = NW + NA;
+  // wavefront w loads chunks w, w + 4, ... of each
+  constexpr int NW = BN / 32, NA = BM / 32, CHUNKS = NW + NA;
   constexpr int STAGE = (BM + BN) * KC;
   constexpr int NST = TWO ? 2 : deep_stages(KIND == KIND_MX, BM, BN);
   // The software pipeline over a step's 32-row blocks: a block's operands are read during the block before it, and the
@@ -98,14 +97,11 @@ __global__ __launch_bounds__(256, TWO ? 2 : 1) void conv_deep_kernel(const DeepA
   // staged rows of this lane: chunk c holds rows 8 c + lane / 8; LDS slot lane % 8 of row r holds K segment
   // (lane % 8) ^ ((r / 2) % 8), the same for all of this wavefront's chunks (they have one parity)
   const int seg = (lane & 7) ^ (lane >> 4) ^ (4 * (wave & 1));
-  auto a_chunk = [&](int i) __attribute__((always_inline)) {
-    return wave + 4 * i - (ACH % 4 != 0 && i == NA - 1 ? (wave & 2) : 0);
-  };
   int x_base[NA];
   uint32_t x_dead[NA];  // bit t: tap t of this row lies outside the image (or past the filter)
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
-    const int m = m0 + 8 * a_chunk(i) + (lane >> 3);
+    const int m = m0 + 8 * (wave + 4 * i) + (lane >> 3);
     const int mc = m < a.M ? m : 0;
     const int q = div_magic(mc, d.wo_mul, d.wo_shift);
     const int ow = mc - q * a.Wo;
@@ -157,7 +153,7 @@ __global__ __launch_bounds__(256, TWO ? 2 : 1) void conv_deep_kernel(const DeepA
       const uint32_t off = (uint32_t)(x_base[i - NW] + xk) | ((x_dead[i - NW] << xsh) & OOB);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.x), (short)0, x_nrec, 0x00020000),
-          (lds_void_t*)(st + (BN / 8 + a_chunk(i - NW)) * 1024), 16, off, 0, 0, 0);
+          (lds_void_t*)(st + (BN / 8 + wave + 4 * (i - NW)) * 1024), 16, off, 0, 0, 0);
     }
   };
 
@@ -332,8 +328,8 @@ __global__ __launch_bounds__(256, TWO ? 2 : 1) void conv_deep_kernel(const DeepA
 #pragma unroll
     for (int j = 0; j < L; ++j)
       mfma_block(MAIN + j, xt[j], wf[s], s, [&](int k) __attribute__((always_inline)) {
-        if (j == 0) {
-constexpr int PER = 16 / SL;  // past the last step: zeros, unused
+        if (j == 0) {  // (past the last step: zeros, unused)
+          constexpr int PER = 16 / SL;
 #pragma unroll
           for (int n = PER * k; n < PER * k + PER; ++n)
             if (n < FIRST_READS) first_read(nxt, s1, n);
@@ -440,8 +436,7 @@ constexpr int PER = 16 / SL;  // past the last step: zeros, unused
     if constexpr (MBW > GB) group(std::integral_constant<int, GB>{}, res, staged);
     if constexpr (MBW > 2 * GB) group(std::integral_constant<int, 2 * GB>{}, res, staged);
     if constexpr (MBW > 3 * GB) group(std::integral_constant<int, 3 * GB>{}, res, staged);
-    if constexpr (MBW > 4 * GB) group(std::integral_constant<int, 4 * GB>{}, res, staged);
-    static_assert(MBW <= 5 * GB, "five groups");
+    static_assert(MBW <= 4 * GB, "four groups");
   };
   using Y = std::integral_constant<bool, true>;
   using N = std::integral_constant<bool, false>;
