@@ -22,9 +22,12 @@ CSRC = PACKAGE / "csrc"
 BUILD = PACKAGE / "_build"
 LIBRARY = PACKAGE / "libflashim_amd.so"
 HOST_LIBRARY = PACKAGE / "libfim_host.so"
-DEVICE_SOURCES = ("quantize.hip", "igemm.hip", "deep_plan.hip", "deep_int8.hip", "deep_mx.hip", "depthwise.hip", "dwpw.hip", "mlp.hip", "stem.hip", "pointwise.hip", "version.hip")
+DEVICE_SOURCES = (
+    "quantize.hip", "igemm.hip", "deep_plan.hip", "deep_int8.hip", "deep_mx.hip", "depthwise.hip", "dwpw.hip", "mlp.hip",
+    "stem.hip", "pointwise.hip", "version.hip",
+)
 PROBE_LIBRARY = PACKAGE / "libflashim_amd_probe.so"
-PROBE_SOURCES = ("probe.hip",)
+PROBE_SOURCES = ("probe.hip", "deep_plan.hip")
 TORCH_LIBRARY = PACKAGE / "libflashim_amd_torch.so"
 ARCH = os.environ.get("FLASHIM_AMD_ARCH", "gfx950")
 HIP_FLAGS = (
@@ -71,7 +74,7 @@ def build(jobs: int = 6) -> Path:
     ``libfim_host.so``. Always rebuilds."""
     BUILD.mkdir(exist_ok=True)
     compiler = hipcc()
-    sources = DEVICE_SOURCES + PROBE_SOURCES
+    sources = tuple(dict.fromkeys(DEVICE_SOURCES + PROBE_SOURCES))
     objects = {src: BUILD / (src.rsplit(".", 1)[0] + ".o") for src in sources}
     commands = [[compiler, *HIP_FLAGS, "-c", str(CSRC / src), "-o", str(objects[src])] for src in sources]
     with ThreadPoolExecutor(max_workers=jobs) as pool:

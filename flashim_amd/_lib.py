@@ -72,6 +72,7 @@ PROBE_SIGNATURES: dict[str, list] = {
     "fim_test_mfma_peak": [_i32, _i64, _i32, _vp, _vp],
     "fim_test_bf16": [_vp, _i64, _vp, _vp],
     "fim_test_gelu": [_vp, _i64, _vp, _vp],
+    "fim_test_deep_plan": [_i32] + [_i64] * 5 + [_i32] * 10 + [_vp],
 }
 
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}

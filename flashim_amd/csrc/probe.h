@@ -29,6 +29,13 @@ int fim_test_mx_exponent(const float* amax, int64_t n, int8_t* out, hipStream_t 
  * 2: INT8 32x32x32 (65536 OP each). out: FP32 [blocks * 256], one sum per thread. */
 int fim_test_mfma_peak(int kind, int64_t blocks, int iters, float* out, hipStream_t stream);
 
+/* The deep convolution kernel's plan for a launch with aligned operands (deep_plan.h), on the current device's CU count
+ * (256 without a device): plan = {wavefronts across the columns (0: not taken), 32-row blocks per wavefront, ragged
+ * channels, two workgroups per CU}. kind 0: INT8, 1: MXFP8; out_mode 0: BF16, 1: INT8, 2: E4M3; residual: a BF16 one laid
+ * out as the output. Runs on the host only. */
+int fim_test_deep_plan(int kind, int64_t B, int64_t H, int64_t W, int64_t Cin, int64_t Cout, int kh, int kw, int sh, int sw,
+                       int ph, int pw, int dh, int dw, int out_mode, int residual, int* plan);
+
 #ifdef __cplusplus
 }
 #endif

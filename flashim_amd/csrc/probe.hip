@@ -3,6 +3,7 @@
 // against torch on the GPU), and an MFMA throughput microbenchmark (the measured peaks the roofline fractions are also
 // quoted against). Declarations: probe.h.
 #include "common.h"
+#include "deep_plan.h"
 #include "probe.h"
 
 namespace fim {
@@ -118,6 +119,33 @@ int fim_test_mfma_peak(int kind, int64_t blocks, int iters, float* out, hipStrea
   else
     mfma_peak_kernel<2><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(iters, out);
   return launch_status();
+}
+
+int fim_test_deep_plan(int kind, int64_t B, int64_t H, int64_t W, int64_t Cin, int64_t Cout, int kh, int kw, int sh, int sw,
+                       int ph, int pw, int dh, int dw, int out_mode, int residual, int* plan) {
+  if (plan == nullptr || sh <= 0 || sw <= 0 || Cin <= 0 || Cout <= 0) return FIM_ERR_INVALID;
+  ConvArgs a = {};
+  a.x = a.w = reinterpret_cast<const uint8_t*>(4096);  // only the alignment is looked at
+  a.out = reinterpret_cast<void*>(4096);
+  a.B = (int)B; a.H = (int)H; a.W = (int)W; a.Cin = (int)Cin; a.Cout = (int)Cout;
+  a.kh = kh; a.kw = kw; a.sh = sh; a.sw = sw; a.ph = ph; a.pw = pw; a.dh = dh; a.dw = dw;
+  a.Ho = (a.H + 2 * ph - dh * (kh - 1) - 1) / sh + 1;
+  a.Wo = (a.W + 2 * pw - dw * (kw - 1) - 1) / sw + 1;
+  a.M = a.B * a.Ho * a.Wo;
+  a.out_mode = out_mode;
+  a.out_ld = a.Cout;
+  if (residual) {
+    a.residual = a.out;
+    a.res_dtype = FIM_BF16;
+    a.res_channels = a.Cout;
+    a.rs_c = 1;
+    a.rs_w = a.Cout;
+    a.rs_h = (int64_t)a.Wo * a.Cout;
+    a.rs_b = (int64_t)a.Ho * a.Wo * a.Cout;
+  }
+  const DeepPlan p = deep_plan(a, kind);
+  plan[0] = p.wn; plan[1] = p.mbw; plan[2] = p.rag; plan[3] = p.two;
+  return FIM_OK;
 }
 
 }  // extern "C"
