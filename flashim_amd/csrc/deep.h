@@ -8,11 +8,12 @@
 // its waits, so they are taken out of the K loop: loads go to LDS two steps ahead (one for the tiles whose three stages
 // do not fit), operands are read one block ahead, the last blocks' MFMAs run past the step's barrier, and reads and loads
 // sit between the MFMAs. K is walked in 16-byte segments across the taps, so only the last step is padded (a Cin of 160
-// takes 12 steps of a 3 x 3 filter instead of 18), and INT8 inputs and outputs of any multiple of 4 channels are taken.
+// takes 12 steps of a 3 x 3 filter instead of 18), and INT8 channel counts may be any multiple of 4 (from 36 in and 68
+// out on).
 // Measured (MI355X): a 160 x 256 step 1570 clocks for 1280 of MFMA issue, at the 1.75 to 1.9 GHz that the matrix cores'
-// power draw leaves; prologue 3.3 us, epilogue 3 to 6 us. INT8 512 -> 512 3 x 3 at 112 x 150 75 -> 45 us (160 x 256
-// tiles), MXFP8 256 -> 256 at 224 x 300 67 -> 49 us (the same), INT8 196 -> 128 at 448 x 600 970 -> 108 to 118 us (two
-// 128 x 128 workgroups per CU; it ran on byte loads).
+// power draw leaves; prologue 3.3 us, epilogue 3 to 6 us. INT8 512 -> 512 3 x 3 at 112 x 150 75 -> 41 to 45 us (160 x 256
+// tiles), MXFP8 256 -> 256 at 224 x 300 67 -> 46 to 49 us (the same), INT8 196 -> 128 at 448 x 600 970 -> 108 to 118 us
+// (two 128 x 128 workgroups per CU; it ran on byte loads).
 #pragma once
 
 #include "deep_plan.h"

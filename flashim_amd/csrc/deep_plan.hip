@@ -18,9 +18,13 @@ static double step_clocks(int wn, int bm, int bn, bool three_stages) {
 // where that is below the estimate for the 128-row kernels, which run without its prologue and epilogue costs (about
 // 8 us a round of tiles, one workgroup per CU) but at half its rate. Their time, in clocks of 1.85 GHz, is 4 us and per
 // 128-byte K step 1.65 us a round of 512 tiles (0.45 to 1.5 us for launches of fewer than 256, which run as 64 x 64
-// tiles; 13.5 us a round, at least 6, where Cin is no multiple of 16: byte loads). Measured, deep
-// against 128-row: INT8 512 -> 512 at 112 x 150 49 / 75 us, MXFP8 256 -> 256 at 224 x 300 50 / 67 us, INT8 196 -> 128 at
-// 448 x 600 108 / 970 us; one-step 1 x 1 layers the other way round (64 -> 256 at 233 x 286 23 / 21 us).
+// tiles; 13.5 us a round, at least 6, where Cin is no multiple of 16: byte loads). Measured, deep against 128-row: INT8
+// 512 -> 512 at 112 x 150 41 to 45 / 75 us, MXFP8 256 -> 256 at 224 x 300 46 to 49 / 67 us, INT8 196 -> 128 at 448 x 600
+// 108 to 118 / 970 us; one-step 1 x 1 layers the other way round (64 -> 256 at 233 x 286 23 / 21 us).
+// The 128-row kernels are the only alternative that is estimated, also where the wide kernel would take the launch instead
+// of them; 1 x 1 launches that fit the pointwise kernels never come here (those kernels are asked first). Cout up to 64
+// fills half of the narrowest tile at most, and a Cin below 36 was not tried (the walk needs two segments a tap, more than
+// 16 channels): both stay with the 128-row kernels, on byte loads where ragged.
 DeepPlan deep_plan(const ConvArgs& a, int kind) {
   const DeepPlan none = {0, 0, false, false};
   const bool mx = kind == KIND_MX;

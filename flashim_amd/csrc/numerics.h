@@ -177,10 +177,10 @@ FIM_HD int8_t quantize_int8_value(float x, float scale) {
 
 // x / s as one multiply and two FMAs, for the INT8 rounding: q0 = x inv (inv = RN(1 / s)) clamped to +-256, the remainder
 // x - q0 s (exact where q0 is within 2 ulp of the quotient), and the corrected quotient. Its rounding to an integer,
-// saturated to +-127, equals that of the IEEE division x / s: checked on the host for every BF16 x against 3000 random
-// scales and nice ones (0.04, 0.5, ..., 1e-38, 3e38), infinities included, and for 2e8 FP32 x on and up to 3 ulp around
-// half-integer multiples of random scales. The clamp keeps infinite and huge quotients out of the remainder (they
-// saturate either way); a NaN stays one. Where the scale's magnitude is below 2^-100 the remainder could underflow: there
+// saturated to +-127, equals that of the IEEE division x / s: the host tests check every BF16 x, infinities included, and
+// the FP32 values up to 3 ulp around every half-integer multiple, for 500 random scales and for nice ones (0.04, 0.5, ...,
+// 1e-38, 3e38). The clamp keeps infinite and huge quotients out of the remainder (they saturate either way); a NaN stays
+// one. Where the scale's magnitude is below 2^-100 the remainder could underflow: there
 // the operands go in scaled by 2^64 (int8_quotient_tiny; values that overflow saturate as well).
 FIM_HD float int8_quotient(float x, float scale, float inv) {
   float q0 = x * inv;
@@ -206,9 +206,9 @@ FIM_HD float int8_quotient_tiny(float x, float scale, float inv) {
 // even) on the grid of unit spacing where M sits, so its low mantissa bits hold rint(x * inv) and its low byte is the
 // INT8 code in two's complement; r = f - M (exact) is the rounded quotient and fma(x, inv, -r) the exact residual, and
 // |residual| >= 0.5 - 2^-15 marks a near-tie. The correction sits behind one wave-uniform branch for all N values (taken
-// when any lane is near a tie), so it does not split the code that produces the inputs, and has no branch of its own:
-// BF16 values over a scale such as 0.04 or 0.5 meet exact ties in nearly every batch (an IEEE division behind a branch
-// per value there made up 40% of the VGG stem's time). The
+// when any lane is near a tie), so it does not split the code that produces the inputs, and has no branch of its own: BF16
+// values over a scale such as 0.04 or 0.05 meet exact ties in nearly every batch, where an IEEE division behind a branch
+// per value cost the VGG stem 11 to 20 us of 45 to 54 (over amax / 127, in 5% of its batches, next to nothing). The
 // saturation is one v_med3_f32 between M - 127 and M + 127 (LO = 0 folds a preceding ReLU in: relu then quantize
 // equals clamping the rounded quotient at 0), so no conversion to an integer is needed: q[i] holds the clamped value's
 // bit pattern, whose low byte is the code (callers keep that byte). 5 VALU operations per value (FMA, subtraction,

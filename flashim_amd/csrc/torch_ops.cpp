@@ -2,7 +2,8 @@
 // allocator, makes one C call on the current stream of its input's device and raises on a nonzero status. Registered in
 // C++, an eager call takes torch's C++ dispatcher only (a Python custom op costs about 10 us a call on the host, more
 // than a small layer's kernel); the fakes stay in library.py. Arguments arrive normalized by the Python impls (dtypes,
-// contiguity, devices); 1-byte float formats cross as their uint8 views.
+// contiguity, devices); 1-byte float formats cross as they are or as their uint8 views (the bodies read bytes), and come
+// back as uint8.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>

@@ -137,7 +137,7 @@ def int8_conv2d_maxpool(x, weight, a_scale, w_scale, bias, kh, kw, sh, sw, ph, p
 @_fake
 def mxfp8_conv2d(x, channel_exponent, weight, weight_exponent, bias, kh, kw, sh, sw, ph, pw, dh, dw, relu, gelu,
                  residual, out_exponent):
-    """``x`` / ``weight``: the ``uint8`` views of E4M3 tensors; E4M3 output (``uint8``) with ``out_exponent``."""
+    """``x`` / ``weight``: E4M3 tensors or their ``uint8`` views; E4M3 output (``uint8``) with ``out_exponent``."""
     b, h, w, _ = x.shape
     ho, wo = conv_out_hw(h, w, kh, kw, sh, sw, ph, pw, dh, dw)
     return x.new_empty((b, ho, wo, weight.shape[0]),
@@ -173,7 +173,7 @@ def im2col_gather(x, kh, kw, sh, sw, ph, pw, dh, dw):
 
 @_fake
 def refiner_mlp(kind, semantics, x, x_scale, w1, w1_scale, b1, h_scale, w2, w2_scale, b2, residual):
-    """The fused 64 -> 256 -> 64 MLP over ``x`` (``uint8`` view) ``[rows, 64]`` -> BF16 ``[rows, 64]``."""
+    """The fused 64 -> 256 -> 64 MLP over ``x`` (INT8 or E4M3) ``[rows, 64]`` -> BF16 ``[rows, 64]``."""
     return x.new_empty((x.shape[0], w2.shape[0]), dtype=torch.bfloat16)
 
 

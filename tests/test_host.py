@@ -193,6 +193,28 @@ def test_host_int8_quotient_rounds_as_the_division(scale):
     assert np.array_equal(got, (x / s).round().clamp(-127, 127).to(torch.int8).numpy())
 
 
+def test_host_int8_quotient_at_random_scales():
+    """The same for 500 scales of either sign from 2^-120 to 2^126, fractions all ones and all zeros among them, and FP32
+    values up to 3 units in the last place around every half-integer multiple."""
+    h = _lib.load_host()
+    rng = np.random.default_rng(0)
+    bits = (rng.integers(7, 254, 500, dtype=np.uint32) << 23) | rng.integers(0, 1 << 23, 500, dtype=np.uint32)
+    bits[:20] |= 0x7FFFFF
+    bits[20:40] &= 0xFF800000
+    scales = bits.view(np.float32) * rng.choice(np.float32([1, -1]), 500)
+    bf16 = (np.arange(65536, dtype=np.uint32) << 16).view(np.float32)
+    bf16 = bf16[~np.isnan(bf16)]
+    for scale in scales:
+        ties = ((np.arange(-130, 130) + 0.5) * np.float64(scale)).astype(np.float32)
+        steps = np.arange(-3, 4, dtype=np.int32)[:, None]
+        near = (ties.view(np.int32)[None] + steps).view(np.float32).ravel()
+        x = np.concatenate([bf16, near[np.isfinite(near)]])
+        with np.errstate(over="ignore", under="ignore"):
+            want = np.clip(np.rint(x / scale), -127, 127).astype(np.int8)
+        got = _call(h.fim_host_int8_quotient, x, np.int8, ctypes.c_float(scale))
+        assert np.array_equal(got, want), scale
+
+
 # -- what an installed package holds and how it loads ----------------------------------------------------------------
 
 
